@@ -15,6 +15,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -122,6 +123,18 @@ __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, void* 
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
                "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(off), "s"(base), "s"(la) : "memory");
+}
+
+// The same with the LDS address given as a uniform byte address plus a constant, and M0 left
+// changed: three instructions instead of six where a loop issues many.  The compiler keeps nothing
+// in M0 (it is not allocatable, and no other instruction of these kernels reads it).
+template <int IMM>
+__device__ __forceinline__ void lds_dma16_at(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               : : "v"(off), "s"(base), "s"(lds), "i"(IMM) : "memory", "scc");
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 
 // RoPE on one interleaved pair with the rounding of eager fp16 ops: each product rounded to

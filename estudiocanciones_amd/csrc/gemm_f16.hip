@@ -13,18 +13,24 @@
 // of half h hold row l & 15, k = 64c + 16 (l >> 4) + 8h .. +7 (ecd_pack_f16), so one 16-byte
 // LDS read is an MFMA A fragment.  The activations x are the B operand.
 //
-// Tiling (template): 4 waves as WN x WM; wave (wn, wm) owns FT 16-feature tiles and RT 16-row
-// tiles of v_mfma_f32_16x16x32_f16, so a block covers BN = 16 WN FT features x BM = 16 WM RT
-// rows.  K advances in 64-wide chunks that go straight from global memory into an NS-stage LDS
-// ring (LDS DMA, no register staging); x rows are stored with their 16-byte pieces XOR-swizzled
-// by row (piece p of row r at position p ^ (r & 7)) so the fragment reads spread over banks.
-// At the top of step c each wave waits until its own loads of chunk c have landed (vmcnt counts
-// the later chunks still allowed in flight), a barrier publishes the chunk and frees the stage
-// read in step c - 1, and then the loads of chunk c + NS - 1 go into that stage.
+// Tiling (template): NW = WN x WM waves; wave (wn, wm) owns FT 32-feature tiles and RT 32-row tiles
+// of v_mfma_f32_32x32x16_f16, so a block covers BN = 32 WN FT features x BM = 32 WM RT rows.  (At
+// one wave per SIMD independent 32x32x16 products issued back to back reach 2.14 PFLOP/s on this
+// chip, 16x16x32 ones 1.86.)  K advances in 64-wide chunks that go straight from global memory into
+// an NS-stage LDS ring (LDS DMA, no register staging); x rows are stored with their 16-byte pieces
+// XOR-swizzled by row (piece p of row r at position p ^ ((r >> 1) & 7)), so that the 16 rows that a
+// ds_read_b128 serves at a time lie in distinct banks (no conflicts counted).
 //
-// Why the shapes: every block re-reads its weight tile and x tile from L2 once per chunk, so the
-// block tile sets the FLOPs per L2 byte (128 x 128: 64 FLOP/B; 256 x 128: 85 FLOP/B), while the
-// number of blocks must still fill 256 CUs; the host picks the tile per shape.
+// What bounds it: a CU takes about 57 bytes per clock through its vector memory path (measured, L2
+// hits), so a block tile needs a high ratio of products to bytes: 128 x 128 needs 575 clocks of
+// loads for 512 of MFMA per chunk, 256 x 256 1150 for 2048.  Loads that miss L2 take 1 to 2 us, so a
+// small tile needs many chunks in flight: NS is what the LDS holds.  Fragments are read half a chunk
+// ahead, interleaved with the products; each DMA takes three instructions (computing every address
+// on the scalar unit took twelve, and the issue slots of a third of the loop).  The output goes through
+// LDS (see the epilogue).  us before -> now, M = 1488 (N, K): (4608, 1536) 31.8 -> 25.7, (8192, 1536)
+// 56.3 -> 41.5, (1536, 1536) 16.6 -> 14.1, (1536, 4096) 36.3 -> 28.2, (9216, 3072) 102 -> 80,
+// (16384, 3072) 182 -> 145, (3072, 8192) 111 -> 84; M = 187: (4608, 1536) 19.8 -> 9.9,
+// (1536, 4096) 26.1 -> 14.4, (3072, 8192) 99.7 -> 36.8; 8192^3 0.90 -> 1.21 PFLOP/s.
 //
 // Block order is XCD-aware: the row blocks that share a weight tile get block ids equal modulo 8,
 // so they run on one XCD and share its L2 (feature blocks in whole groups of 8; the grid has
@@ -47,49 +53,34 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
 // 0 .. MAXL) stay in flight; PER instructions per chunk; LGKM: also drain LDS operations
 template <int PER, int MAXL, bool LGKM>
 __device__ __forceinline__ void wait_chunk(int later) {
-  if constexpr (MAXL >= 3) {
-    if (later >= 3) { if constexpr (LGKM) wait_vm_lgkm0<3 * PER>(); else wait_vm<3 * PER>(); return; }
-  }
-  if constexpr (MAXL >= 2) {
-    if (later >= 2) { if constexpr (LGKM) wait_vm_lgkm0<2 * PER>(); else wait_vm<2 * PER>(); return; }
-  }
   if constexpr (MAXL >= 1) {
-    if (later >= 1) { if constexpr (LGKM) wait_vm_lgkm0<PER>(); else wait_vm<PER>(); return; }
+    if (later < MAXL) {
+      wait_chunk<PER, MAXL - 1, LGKM>(later);
+      return;
+    }
   }
-  if constexpr (LGKM) wait_vm_lgkm0<0>(); else wait_vm0();
+  if constexpr (LGKM) wait_vm_lgkm0<MAXL * PER>(); else wait_vm<MAXL * PER>();
 }
 
-// A fragments (two k-halves) of the wave's FT weight tiles and B fragments of its RT row tiles
-// for one chunk of LDS stage (lw_st, lx_st).
-template <int FT, int RT>
-__device__ __forceinline__ void f16_frags(const f16* lw_st, const f16* lx_st, int wn, int wm,
-                                          int lane, f16x8 (&wa)[FT], f16x8 (&wb)[FT],
-                                          f16x8 (&fa)[RT], f16x8 (&fb)[RT]) {
-  const int sw = lane & 7, p0 = 2 * (lane >> 4);
-#pragma unroll
-  for (int ft = 0; ft < FT; ++ft) {
-    const f16* tp = lw_st + (wn * FT + ft) * 1024;
-    wa[ft] = *(const f16x8*)(tp + 8 * lane);
-    wb[ft] = *(const f16x8*)(tp + 512 + 8 * lane);
-  }
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const f16* xr = lx_st + ((wm * RT + rt) * 16 + (lane & 15)) * 64;
-    fa[rt] = *(const f16x8*)(xr + 8 * (p0 ^ sw));
-    fb[rt] = *(const f16x8*)(xr + 8 * ((p0 + 1) ^ sw));
+template <int I>
+struct IC {
+  static constexpr int value = I;
+};
+// f(IC<B>{}), .., f(IC<E - 1>{})
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(IC<B>{});
+    static_for<B + 1, E>(f);
   }
 }
 
-// acc[ft][rt] += w[ft] x f[rt] over one k-half; consecutive MFMAs write different accumulators
+// The fragments of half a 64-wide chunk, two k-steps of v_mfma_f32_32x32x16_f16: lane l holds
+// feature (or row) l & 31 of a 32-wide tile, k = 16 s + 8 (l >> 5) .. + 7 of step s.
 template <int FT, int RT>
-__device__ __forceinline__ void f16_mfma_half(f32x4 (&acc)[FT][RT], const f16x8 (&w)[FT],
-                                              const f16x8 (&f)[RT]) {
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-      acc[ft][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[ft], f[rt], acc[ft][rt], 0, 0, 0);
-}
+struct Frags {
+  f16x8 w[2][FT], x[2][RT];
+};
 
 // Row layouts of a convolution as a GEMM over implicit tap columns (the waveform decoder):
 // row m = b * T + t of the GEMM.  With k > 0, x is time-major with xpad zero rows before each
@@ -110,27 +101,30 @@ struct RopeOut {
   int T, H, HD;
 };
 
-__device__ __forceinline__ long seq_row(long m, int T, int pad) {
-  const long b = m / T;
-  return b * (T + pad) + pad + (m - b * T);
+__device__ __forceinline__ long seq_row(int m, int T, int pad) {
+  const int b = m / T;
+  return (long)b * (T + pad) + pad + (m - b * T);
 }
 
-// 128 x 128 tiles are built for two waves per SIMD (two blocks per CU); the larger ones for one
-template <int EPI, int WN, int WM, int FT, int RT, int NS, bool PL>
-__global__ __launch_bounds__(256, (FT * RT <= 16 ? 2 : 1)) void gemm_f16w_kernel(
+// piece p of x row r lies at position p ^ x_swz(r) of its 128 bytes
+__device__ __forceinline__ int x_swz(int r) { return (r >> 1) & 7; }
+
+template <int EPI, int WN, int WM, int FT, int RT, int NS>
+__global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
     const f16* __restrict__ x, long ldx, const f16* __restrict__ wp,
     const float* __restrict__ bias, float alpha, const f16* res, long ldr,
     f16* y, long ldy, int M, int N, int K, int nfb, int nmb, RowMap rm,
     RopeOut ro) {
-  static_assert(WN * WM == 4, "four waves");
-  constexpr int BN = 16 * WN * FT;      // features per block
-  constexpr int BM = 16 * WM * RT;      // rows per block
-  constexpr int WI = BN / 16 * 2 / 4;   // weight DMA instructions per wave per chunk (1 KB each)
-  constexpr int XI = BM / 8 / 4;        // x DMA instructions per wave per chunk (8 rows each)
+  constexpr int NW = WN * WM;           // waves
+  constexpr int BN = 32 * WN * FT;      // features per block
+  constexpr int BM = 32 * WM * RT;      // rows per block
+  constexpr int WI = BN / 8 / NW;       // weight DMA instructions per wave per chunk (1 KB each)
+  constexpr int XI = BM / 8 / NW;       // x DMA instructions per wave per chunk (8 rows each)
   constexpr int PER_CHUNK = WI + XI;
-  static_assert(NS >= 2 && NS <= 4 && PER_CHUNK * (NS - 1) < 64, "vmcnt range");
-  __shared__ __align__(16) f16 lw[NS][BN / 16 * 1024];  // BN / 16 tiles x 2 KB
-  __shared__ __align__(16) f16 lx[NS][BM * 64];         // BM rows x 128 B
+  static_assert(WI * 8 * NW == BN && XI * 8 * NW == BM, "whole DMA instructions per wave");
+  static_assert(NS >= 2 && PER_CHUNK * (NS - 1) < 64, "vmcnt range");
+  constexpr int LW = BN * 64, LX = BM * 64, STG = LW + LX;  // halfs per stage
+  __shared__ __align__(16) f16 lds[NS * STG];
 
   // feature blocks in full groups of 8 share XCDs with their row blocks; the remaining
   // nfb % 8 feature blocks (all of them when nfb < 8) are laid out row-major after them
@@ -160,200 +154,247 @@ __global__ __launch_bounds__(256, (FT * RT <= 16 ? 2 : 1)) void gemm_f16w_kernel
   const long tile_bytes = (long)nch * 2048;
 
   // DMA sources: weight instruction j of this wave is tile t = i >> 1, half h = i & 1 with
-  // i = wv + 4 j (tiles past N re-read the last tile; their results are never stored); x
-  // instruction j covers rows 8 i .. 8 i + 7, i = wv + 4 j (rows past M re-read row M - 1).
-  const char* wsrc[WI];
-  int wdst[WI];
+  // i = wv + NW j (tiles past N re-read the last tile; their results are never stored); x
+  // instruction j covers rows 8 i .. 8 i + 7, i = wv + NW j (rows past M re-read row M - 1).
+  // Every address is a uniform base, advanced per chunk, plus a per-lane offset.
+  const int t0 = min(n0 / 16, ntiles - 1);
+  const char* wb = (const char*)wp + (long)t0 * tile_bytes;
+  uint32_t woff[WI];
 #pragma unroll
   for (int j = 0; j < WI; ++j) {
-    const int i = wv + 4 * j;
-    const int t = i >> 1, h = i & 1;
-    wsrc[j] = (const char*)wp + (long)min(n0 / 16 + t, ntiles - 1) * tile_bytes + 1024 * h;
-    wdst[j] = t * 1024 + 512 * h;  // in halfs
+    const int i = wv + NW * j;
+    woff[j] = (uint32_t)((min(n0 / 16 + (i >> 1), ntiles - 1) - t0) * tile_bytes) + 1024 * (i & 1) + 16 * lane;
   }
-  const uint32_t woff = 16u * lane;
-  const int xpiece = (lane & 7) ^ (lane >> 3);
   // with a 2x row-repeat (rm.rep == 2) output step t reads source row (t + o) >> 1 for tap o:
   // (t >> 1) + (o >> 1) for even o, ((t + 1) >> 1) + (o >> 1) for odd o -- two lane rows
   uint32_t xoff[XI], xoff1[XI];
 #pragma unroll
   for (int j = 0; j < XI; ++j) {
-    const int i = wv + 4 * j;
-    long xr = min(m0 + 8 * i + (lane >> 3), M - 1), xr1 = xr;
+    const int i = wv + NW * j;
+    const int xpiece = (lane & 7) ^ x_swz(8 * i + (lane >> 3));
+    const int row = min(m0 + 8 * i + (lane >> 3), M - 1);
+    long xr = row, xr1 = row;
     if (rm.k && rm.rep == 2) {
-      const long b = xr / rm.T, t = xr - b * rm.T;
-      const long base = b * (rm.T / 2 + rm.xpad) + rm.xpad;
+      const int b = row / rm.T, t = row - b * rm.T;
+      const long base = (long)b * (rm.T / 2 + rm.xpad) + rm.xpad;
       xr = base + (t >> 1);
       xr1 = base + ((t + 1) >> 1);
     } else if (rm.k) {
-      xr = xr1 = seq_row(xr, rm.T, rm.xpad);
+      xr = xr1 = seq_row(row, rm.T, rm.xpad);
     }
     xoff[j] = (uint32_t)(xr * ldx * 2 + 16 * xpiece);
     xoff1[j] = (uint32_t)(xr1 * ldx * 2 + 16 * xpiece);
   }
-  // chunk c's x base: plain K offset 64 c, or tap j = c / cpt shifted by off[j] rows (by
-  // off[j] >> 1 with a 2x row-repeat, odd taps reading the second set of lane rows)
-  auto issue = [&](int c, int st) {
-#pragma unroll
-    for (int j = 0; j < WI; ++j) lds_dma16(wsrc[j] + (long)c * 2048, woff, &lw[st][wdst[j]]);
-    const f16* xb = x + (long)c * 64;
-    bool odd = false;
-    if (rm.k) {
-      const int tj = c / rm.cpt;
-      int o = rm.off[0];
-#pragma unroll
-      for (int i = 1; i < 8; ++i)
-        if (tj == i) o = rm.off[i];
-      odd = rm.rep == 2 && (o & 1);
-      xb = x + (long)(rm.rep == 2 ? (o >> 1) : o) * ldx + (long)(c - tj * rm.cpt) * 64;
+  // x base of the next chunk to load: plain K offset 64 c, or tap j = c / cpt shifted by off[j]
+  // rows (by off[j] >> 1 with a 2x row-repeat, odd taps reading the second set of lane rows)
+  const f16* xb = x;
+  int tap = 0, tc = 0;
+  bool odd = false;
+  auto set_tap = [&]() {
+    const int o = rm.off[tap];
+    odd = rm.rep == 2 && (o & 1);
+    xb = x + (long)(rm.rep == 2 ? (o >> 1) : o) * ldx;
+  };
+  if (rm.k) set_tap();
+  auto next_chunk = [&]() {
+    xb += 64;
+    wb += 2048;
+    if (rm.k && ++tc == rm.cpt) {
+      tc = 0;
+      ++tap;
+      if (tap < rm.k) set_tap();
     }
-#pragma unroll
-    for (int j = 0; j < XI; ++j)
-      lds_dma16(xb, odd ? xoff1[j] : xoff[j], &lx[st][8 * (wv + 4 * j) * 64]);
+  };
+  // DMA instruction J of the next chunk into the stage at LDS byte address `sa` (this wave's first
+  // KB of it): weights first, then x rows
+  auto dma = [&](auto J, uint32_t sa) {
+    constexpr int j = decltype(J)::value;
+    if constexpr (j < WI)
+      lds_dma16_at<NW * j * 1024>(wb, woff[j], sa);
+    else
+      lds_dma16_at<LW * 2 + NW * (j - WI) * 1024>(xb, odd ? xoff1[j - WI] : xoff[j - WI], sa);
+  };
+  const uint32_t lds0 = lds_addr(lds) + wv * 1024;
+
+  f32x16 acc[FT][RT];
+  static_for<0, FT * RT>([&](auto I) {
+    acc[I.value / RT][I.value % RT] = (f32x16)(0.f);
+  });
+
+  // fragment addresses within a stage (halfs): a 32-feature tile is two packed 16-row tiles, octet
+  // o = 2 s + (lane >> 5) of k-step s lies in half o & 1 = lane >> 5 at 16-byte unit 16 s + row
+  const int wfo = (wn * FT * 2 + ((lane >> 4) & 1)) * 1024 + (lane >> 5) * 512 + (lane & 15) * 8;
+  int xfo[4];
+  static_for<0, 4>([&](auto S) {
+    xfo[S.value] = LW + (wm * RT * 32 + (lane & 31)) * 64 +
+                   8 * ((2 * S.value + (lane >> 5)) ^ x_swz(lane & 31));
+  });
+
+  // read I of a half chunk's fragments (k-steps 2 H and 2 H + 1), k-step by k-step
+  constexpr int NM = 2 * FT * RT, NR = 2 * (FT + RT);
+  auto read1 = [&](auto I, auto H, const f16* base, Frags<FT, RT>& f) {
+    constexpr int s = decltype(I)::value / (FT + RT), i = decltype(I)::value % (FT + RT);
+    constexpr int ks = 2 * decltype(H)::value + s;
+    if constexpr (i < FT)
+      f.w[s][i] = *(const f16x8*)(base + wfo + 128 * ks + i * 2048);
+    else
+      f.x[s][i - FT] = *(const f16x8*)(base + xfo[ks] + (i - FT) * 2048);
+  };
+  // the products of a half chunk, interleaved with the reads of the next half chunk's fragments
+  // (in the first half of the products, so that they have landed at its end) and, with LOAD, the
+  // loads of a later chunk
+  auto half = [&](const Frags<FT, RT>& f, auto H, const f16* base, Frags<FT, RT>& nf, auto LOAD,
+                  uint32_t sa) {
+    constexpr int RH = NM / 2;
+    static_for<0, NM>([&](auto I) {
+      constexpr int m = decltype(I)::value, s = m / (FT * RT), ft = m % (FT * RT) / RT, rt = m % RT;
+      acc[ft][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.w[s][ft], f.x[s][rt], acc[ft][rt], 0, 0, 0);
+      if constexpr (decltype(LOAD)::value)
+        static_for<m * PER_CHUNK / NM, (m + 1) * PER_CHUNK / NM>([&](auto J) { dma(J, sa); });
+      if constexpr (m < RH)
+        static_for<m * NR / RH, (m + 1) * NR / RH>([&](auto J) { read1(J, H, base, nf); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
   };
 
-  f32x4 acc[FT][RT];
-#pragma unroll
-  for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) acc[ft][rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < NS; ++s)
+    if (s < nch) {
+      static_for<0, PER_CHUNK>([&](auto J) { dma(J, lds0 + s * (STG * 2)); });
+      next_chunk();
+    }
+  wait_chunk<PER_CHUNK, NS - 1, false>(min(NS - 1, nch - 1));
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  Frags<FT, RT> fa, fc;
+  static_for<0, NR>([&](auto I) { read1(I, IC<0>{}, lds, fa); });
 
-  if constexpr (PL) {
-    // Software-pipelined: the fragments of chunk c + 1 are read from LDS while the second
-    // k-half MFMAs of chunk c run, and the wait + barrier for chunk c + 1 sit behind the first
-    // k-half MFMAs, so no MFMA waits for an LDS read at a chunk boundary.  Chunk c + NS goes
-    // into the stage of chunk c (its fragments are in registers by then), so NS - 1 chunks of
-    // DMA stay in flight behind the one being computed.
-    f16x8 wa0[FT], wb0[FT], fa0[RT], fb0[RT], wa1[FT], wb1[FT], fa1[RT], fb1[RT];
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      if (s < nch) issue(s, s);
-    wait_chunk<PER_CHUNK, NS - 1, false>(min(NS - 1, nch - 1));
+  // Chunk c: its first half while its second half is read; then, with chunk c + 1 landed for this
+  // wave (later ones may fly) and its own reads of chunk c done, a barrier that publishes the one and
+  // frees the stage of the other; then the second half while chunk c + 1's first half is read and
+  // chunk c + NS loaded into the stage left free.
+  int c = 0, st = 0;  // st: stage of chunk c
+  for (; c < nch - NS; ++c) {
+    half(fa, IC<1>{}, lds + st * STG, fc, IC<0>{}, 0);
+    wait_vm_lgkm0<(NS - 2) * PER_CHUNK>();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    f16_frags<FT, RT>(lw[0], lx[0], wn, wm, lane, wa0, wb0, fa0, fb0);
-    // one chunk: MFMAs on (wa, wb, fa, fb) = chunk c, next fragments into (na, nb, nfa, nfb)
-#define F16_PL_STEP(c, wa, wb, fa, fb, na, nb, nfa, nfb)                                   \
-    do {                                                                                  \
-      f16_mfma_half<FT, RT>(acc, wa, fa);                                                 \
-      if ((c) + 1 < nch) {                                                                \
-        /* own DMA of c + 1 landed (later chunks may fly), own reads of c done */         \
-        wait_chunk<PER_CHUNK, NS - 2, true>(min(NS - 2, nch - 2 - (c)));                  \
-        asm volatile("" ::: "memory");                                                    \
-        __builtin_amdgcn_s_barrier();                                                     \
-        asm volatile("" ::: "memory");                                                    \
-        if ((c) + NS < nch) issue((c) + NS, (c) % NS);                                    \
-        const int sn = ((c) + 1) % NS;                                                    \
-        f16_frags<FT, RT>(lw[sn], lx[sn], wn, wm, lane, na, nb, nfa, nfb);                \
-      }                                                                                   \
-      f16_mfma_half<FT, RT>(acc, wb, fb);                                                 \
-    } while (0)
-    for (int c = 0; c < nch; c += 2) {
-      F16_PL_STEP(c, wa0, wb0, fa0, fb0, wa1, wb1, fa1, fb1);
-      if (c + 1 < nch) F16_PL_STEP(c + 1, wa1, wb1, fa1, fb1, wa0, wb0, fa0, fb0);
-    }
-#undef F16_PL_STEP
-  } else {
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < nch) issue(s, s);
-  for (int c = 0; c < nch; ++c) {
-    // chunk c landed for this wave: later chunks c + 1 .. c + NS - 2 may still be in flight
-    wait_chunk<PER_CHUNK, NS - 2, false>(min(NS - 2, nch - 1 - c));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();  // chunk c visible to every wave; stage of c - 1 free
-    asm volatile("" ::: "memory");
-    if (c + NS - 1 < nch) issue(c + NS - 1, (c + NS - 1) % NS);
-    const int st = c % NS;
-    f16x8 wa[FT], wb[FT], fa[RT], fb[RT];
-    f16_frags<FT, RT>(lw[st], lx[st], wn, wm, lane, wa, wb, fa, fb);
-    f16_mfma_half<FT, RT>(acc, wa, fa);
-    f16_mfma_half<FT, RT>(acc, wb, fb);
+    const int sn = st + 1 == NS ? 0 : st + 1;
+    half(fc, IC<0>{}, lds + sn * STG, fa, IC<1>{}, lds0 + st * (STG * 2));
+    next_chunk();
+    st = sn;
   }
+  for (; c < nch; ++c) {
+    half(fa, IC<1>{}, lds + st * STG, fc, IC<0>{}, 0);
+    if (c + 1 < nch) {
+      wait_chunk<PER_CHUNK, NS - 2, true>(min(NS - 2, nch - 2 - c));
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    // (behind the last chunk the reads return a stage's old contents, never used)
+    const int sn = st + 1 == NS ? 0 : st + 1;
+    half(fc, IC<0>{}, lds + sn * STG, fa, IC<0>{}, 0);
+    st = sn;
   }
 
-  // epilogue: lane holds features nb .. nb + 3 of row m for every (ft, rt).  Where the rows of
-  // y (and res) are 8-byte aligned the four values go out as one 8-byte store.
-  const bool vec = ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0) &&
-                   (!res || (((ldr & 3) == 0) && (((uintptr_t)res & 7) == 0)));
-  // F16_ROPE: the batch item and time step of each of this lane's row tiles
-  int rb[RT], rtm[RT];
-  if constexpr (EPI == F16_ROPE) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int mm = min(m0 + (wm * RT + rt) * 16 + (lane & 15), M - 1);
-      rb[rt] = mm / ro.T;
-      rtm[rt] = mm - rb[rt] * ro.T;
-    }
-  }
-#pragma unroll
-  for (int ft = 0; ft < FT; ++ft) {
-    const int nb = n0 + (wn * FT + ft) * 16 + 4 * (lane >> 4);
-    if (nb >= N) continue;
-    // F16_ROPE: section (q, k, v), head and offset of this lane's 4 features
-    int sec = 0, hc = 0, hh = 0, d = 0;
-    if constexpr (EPI == F16_ROPE) {
-      const int D = ro.H * ro.HD;
-      sec = nb >= 2 * D ? 2 : (nb >= D ? 1 : 0);
-      hc = nb - sec * D;
-      hh = hc / ro.HD;
-      d = hc - hh * ro.HD;
-    }
-    float bv[4] = {0.f, 0.f, 0.f, 0.f};
+  // Epilogue.  A lane holds features 8 g + 4 (lane >> 5) .. + 3 (g < 4) of row lane & 31 of each of
+  // its tiles.  The rounded sums go through LDS (the stages are free once every wave has read its last
+  // fragments), so that a short loop finishes them in 16-byte pieces of consecutive features and
+  // writes whole row segments.  Unrolled over the accumulators, with 8-byte stores to 32 rows per
+  // instruction, the same work took about 1.1 us per 32 x 32 tile of a wave, most of it instruction
+  // fetch (the code runs once per workgroup).
+  constexpr int PR = BN / 8;                       // 16-byte pieces per row
+  constexpr int SM = PR < 16 ? PR - 1 : 15;
+  auto piece = [](int r, int p) { return (r * PR + (p ^ (r & SM))) * 8; };  // in halfs
+  static_assert(NS * STG >= BM * BN, "the output tile fits the stages");
+  __syncthreads();
+  static_for<0, 4 * FT>([&](auto I) {
+    constexpr int ft = decltype(I)::value >> 2, g = decltype(I)::value & 3;
+    const int nl = (wn * FT + ft) * 32 + 8 * g + 4 * (lane >> 5);
+    f32x4 bv = (f32x4){0.f, 0.f, 0.f, 0.f};
     if (bias) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bv[r] = bias[min(nb + r, N - 1)];
+      for (int r = 0; r < 4; ++r) bv[r] = bias[min(n0 + nl + r, N - 1)];
     }
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int mm = m0 + (wm * RT + rt) * 16 + (lane & 15);
-      if (mm >= M) continue;
-      const long m = rm.ypad >= 0 ? seq_row(mm, rm.T, rm.ypad) : mm;
+    static_for<0, RT>([&](auto R) {
+      constexpr int rt = decltype(R)::value;
+      const int r = (wm * RT + rt) * 32 + (lane & 31);
       f16x4 yv;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        yv[r] = (f16)(acc[ft][rt][r] + bv[r]);
-        if (EPI == F16_PRELU) {
-          if ((float)yv[r] < 0.f) yv[r] = (f16)((float)yv[r] * alpha);  // alpha: the slope
-        } else if (alpha != 1.0f) {
-          yv[r] = (f16)((float)yv[r] * alpha);
+      for (int j = 0; j < 4; ++j) yv[j] = (f16)(acc[ft][rt][4 * g + j] + bv[j]);
+      *(f16x4*)(lds + piece(r, nl >> 3) + (nl & 4)) = yv;
+    });
+  });
+  __syncthreads();
+  // 16-byte rows of y (and res) take one store per piece
+  const bool vec = ((ldy & 7) == 0) && (((uintptr_t)y & 15) == 0) &&
+                   (!res || (((ldr & 7) == 0) && (((uintptr_t)res & 15) == 0)));
+#pragma unroll 1
+  for (int i = tid; i < BM * PR; i += 64 * NW) {
+    const int r = i / PR, p = i - r * PR;
+    const int mm = m0 + r, nb = n0 + 8 * p;
+    if (mm >= M || nb >= N) continue;
+    f16x8 v = *(const f16x8*)(lds + piece(r, p));
+    if constexpr (EPI == F16_STORE || EPI == F16_PRELU) {
+      const long m = rm.ypad >= 0 ? seq_row(mm, rm.T, rm.ypad) : mm;
+      if constexpr (EPI == F16_PRELU) {  // alpha: the slope
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if ((float)v[j] < 0.f) v[j] = (f16)((float)v[j] * alpha);
+      } else if (alpha != 1.0f) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (f16)((float)v[j] * alpha);
+      }
+      if (vec && nb + 7 < N) {
+        if (res) v = v + *(const f16x8*)(res + m * ldr + nb);
+        *(f16x8*)(y + m * ldy + nb) = v;
+      } else {
+        for (int j = 0; j < 8 && nb + j < N; ++j) {
+          f16 o = v[0];
+          if (res) o = o + res[m * ldr + nb + j];
+          y[m * ldy + nb + j] = o;
+          v = __builtin_shufflevector(v, v, 1, 2, 3, 4, 5, 6, 7, 0);
         }
       }
-      if (EPI == F16_STORE || EPI == F16_PRELU) {
-        if (vec && nb + 3 < N) {
-          if (res) yv = yv + *(const f16x4*)(res + (long)m * ldr + nb);
-          *(f16x4*)(y + (long)m * ldy + nb) = yv;
-        } else {
+    } else if constexpr (EPI == F16_ROPE) {
+      // sections q, k, v; 4 features never straddle a head (HD % 4 == 0)
+      const int D = ro.H * ro.HD;
+      const int rb = mm / ro.T, t = mm - rb * ro.T;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            if (nb + r < N) {
-              f16 o = yv[r];
-              if (res) o = o + res[(long)m * ldr + nb + r];
-              y[(long)m * ldy + nb + r] = o;
-            }
-          }
-        }
-      } else if (EPI == F16_ROPE) {  // 4 features never straddle a head (HD % 4 == 0)
-        const int t = rtm[rt];
+      for (int q = 0; q < 2; ++q) {
+        const int n = nb + 4 * q;
+        if (n >= N) break;
+        const int sec = n >= 2 * D ? 2 : (n >= D ? 1 : 0);
+        const int hc = n - sec * D, hh = hc / ro.HD, d = hc - hh * ro.HD;
+        f16x4 o = q ? __builtin_shufflevector(v, v, 4, 5, 6, 7) : __builtin_shufflevector(v, v, 0, 1, 2, 3);
         if (sec < 2) {
           const f16x4 cs = *(const f16x4*)(ro.tab + (long)t * ro.HD + d);  // pairs d/2, d/2 + 1
           f16 o0, o1, o2, o3;
-          rope_pair_f16((float)yv[0], (float)yv[1], (float)cs[0], (float)cs[1], o0, o1);
-          rope_pair_f16((float)yv[2], (float)yv[3], (float)cs[2], (float)cs[3], o2, o3);
-          yv = (f16x4){o0, o1, o2, o3};
+          rope_pair_f16((float)o[0], (float)o[1], (float)cs[0], (float)cs[1], o0, o1);
+          rope_pair_f16((float)o[2], (float)o[3], (float)cs[2], (float)cs[3], o2, o3);
+          o = (f16x4){o0, o1, o2, o3};
         }
-        f16* dst = sec == 0 ? ro.q + m * (ro.H * ro.HD) + hc
-                            : (sec == 1 ? ro.k : ro.v) +
-                                  (((long)rb[rt] * ro.H + hh) * ro.T + t) * ro.HD + d;
-        *(f16x4*)dst = yv;
-      } else {  // (a_j, b_j, a_j+1, b_j+1) with j = nb / 2; N even
-        const int j = nb >> 1;
-        const float a0 = (float)yv[0], a1 = (float)yv[2];
-        f16x2 o;
-        o.x = (f16)(a0 / (1.0f + expf(-a0))) * yv[1];
-        o.y = (f16)(a1 / (1.0f + expf(-a1))) * yv[3];
-        *(f16x2*)(y + (long)m * ldy + j) = o;
+        f16* dst = sec == 0 ? ro.q + (long)mm * D + hc
+                            : (sec == 1 ? ro.k : ro.v) + (((long)rb * ro.H + hh) * ro.T + t) * ro.HD + d;
+        *(f16x4*)dst = o;
+      }
+    } else {  // pairs (a_j, b_j) with j = nb / 2 ..; N even
+      f16x2 o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float a = (float)v[2 * q];
+        const f16 s = (f16)(a / (1.0f + expf(-a))) * v[2 * q + 1];
+        o[q >> 1][q & 1] = s;
+      }
+      f16* dst = y + (long)mm * ldy + (nb >> 1);
+      if (nb + 7 < N && ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0)) {
+        *(f16x4*)dst = (f16x4){o[0].x, o[0].y, o[1].x, o[1].y};
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (nb + 2 * q < N) dst[q] = o[q >> 1][q & 1];
       }
     }
   }
@@ -381,77 +422,85 @@ __global__ __launch_bounds__(256) void pack_f16_kernel(const f16* __restrict__ w
   *(u32x4*)(out + (tile * nch + c) * 1024 + 512 * h + 8 * l) = v;
 }
 
-// Tile configurations: {WN, WM, FT, RT, NS}.
-//   1: 128 x 128, waves 4 x 1 (32 features x 128 rows each), 2 stages, 64 KB LDS
-//   2: 128 x 128, waves 2 x 2 (64 x 64 each), 2 stages, 64 KB
-//   3: 256 x 128, waves 4 x 1 (64 x 128 each), 2 stages, 96 KB
-//   4: 256 x 128, waves 4 x 1, 3 stages, 144 KB
-//   5: 256 x 128, waves 2 x 2 (128 x 64 each), 2 stages, 96 KB
-//   6: 128 x 256, waves 2 x 2 (64 x 128 each), 2 stages, 96 KB
-//   7: 128 x 128, waves 2 x 2, 3 stages, 96 KB
-//   8: as 2, software-pipelined (next chunk's fragments read during this chunk's MFMAs)
-//   9: as 1, software-pipelined
-//  10: 128 x 64, waves 4 x 1 (32 x 64 each), software-pipelined, 48 KB
-//  11: 128 x 64, waves 2 x 2 (64 x 32 each), software-pipelined, 48 KB
-//  12: 64 x 128, waves 1 x 4 (64 x 32 each), software-pipelined, 48 KB (outputs <= 64 wide)
-//  13: 64 x 256, waves 1 x 4 (64 x 64 each), software-pipelined, 80 KB
-//  14: 64 x 64, waves 2 x 2 (32 x 32 each), software-pipelined, 32 KB
-//  15: as 14 with 3 stages, 48 KB
-//  16: 128 x 96, waves 2 x 2 (64 x 48 each), software-pipelined, 56 KB
-template <int EPI, int WN, int WM, int FT, int RT, int NS, bool PL = false>
+template <int EPI, int WN, int WM, int FT, int RT, int NS>
 static int launch_cfg(const f16* x, long ldx, const f16* wp, const float* bias, float alpha,
                       const f16* res, long ldr, f16* y, long ldy, int M, int N, int K,
                       const RowMap& rm, const RopeOut& ro, hipStream_t st) {
-  constexpr int BN = 16 * WN * FT, BM = 16 * WM * RT;
+  constexpr int BN = 32 * WN * FT, BM = 32 * WM * RT;
   const int nfb = (N + BN - 1) / BN;
   const int nmb = (M + BM - 1) / BM;
   const long blocks = (long)nfb * nmb;
   if (blocks > 0x7FFFFFFFL) return ECD_ENOTSUP;
-  hipLaunchKernelGGL((gemm_f16w_kernel<EPI, WN, WM, FT, RT, NS, PL>), dim3((unsigned)blocks),
-                     dim3(256), 0, st, x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, nfb,
-                     nmb, rm, ro);
+  hipLaunchKernelGGL((gemm_f16w_kernel<EPI, WN, WM, FT, RT, NS>), dim3((unsigned)blocks),
+                     dim3(64 * WN * WM), 0, st, x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K,
+                     nfb, nmb, rm, ro);
   return ecd_launch_status();
 }
 
-// Library default per shape (N counts output features before the SiLU pairing).
-static int default_cfg(int M, int N, int K, bool silu) {
-  // blocks of 128 x 128: below 256 (one per CU) or 512 (the two that fit per CU) a smaller block
-  // fills the resident slots that 128 x 128 leaves empty
-  const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (silu) return 8;
-  if (N <= 64) return 12;                            // the decoder's 64-channel convs
-  if (N <= 256 && K >= 4096 && t128 < 256) return 15;  // few blocks, long K: 3 stages in flight
-  if (N <= 1536 && t128 < 256) return 14;            // 64 x 64
-  if (N <= 1536 && t128 < 512) return 10;            // 128 x 64
-  if (N <= 3072 && t128 < 512) return 16;            // 128 x 96
-  if (N <= 1024) return 1;                           // the decoder's wider convs over many rows
-  return 8;
+// The tiles (features x rows, LDS stages).  1 to 8 leave room for one workgroup per CU: a launch takes
+// ceil(blocks / 256) rounds, a round about K / 64 chunk times plus a fill and an epilogue; both in ns,
+// measured over K = 1536 .. 8192 with 100 to 256 workgroups.
+struct Tile {
+  int bn, bm, chunk, edge;
+};
+constexpr Tile TILES[8] = {
+    {256, 256, 1550, 4500},  // 1: 8 waves of 64 x 128, 2 stages
+    {256, 192, 1450, 3500},  // 2: 8 waves of 64 x 96, 2 stages
+    {256, 128, 850, 2500},   // 3: 8 waves of 64 x 64, 3 stages
+    {128, 192, 620, 3000},   // 4: 8 waves of 32 x 96, 3 stages
+    {128, 128, 440, 1200},   // 5: 8 waves of 32 x 64, 4 stages
+    {128, 64, 300, 800},     // 6: 4 waves of 64 x 32, 5 stages
+    {64, 128, 300, 800},     // 7: 4 waves of 32 x 64, 5 stages
+    {64, 64, 220, 600},      // 8: 4 waves of 32 x 32, 8 stages
+};
+// 9: 128 x 128, 8 waves, 2 stages; 10: 64 x 128, 8 waves, 2 stages: several workgroups per CU, for the
+// waveform decoder's convolutions of at most 128 channels over many rows, whose few chunks leave the
+// fill and the stores to be hidden by other workgroups (476160 rows, 128 channels, us for K = 896 / 128:
+// tile 9 213 / 43, 5 228 / 62, 3 270 / 79; 1.4 M rows, 64 channels, K = 448 / 64: tile 10 274 / 69,
+// 9 295 / 91, 7 322 / 134).
+constexpr int MANY_ROWS = 16384;
+
+// Library default per shape (N counts output features before the SiLU pairing): the tile of the
+// shortest estimate.  (Of 29 shapes measured with every tile it is the fastest or within 10% of it.)
+static int default_cfg(int M, int N, int K) {
+  if (M >= MANY_ROWS && N <= 128) return N <= 64 ? 10 : 9;
+  int best = 1;
+  long tb = 0;
+  for (int i = 0; i < 8; ++i) {
+    const Tile& t = TILES[i];
+    const long blocks = (long)((N + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
+    const long est = (blocks + 255) / 256 * ((long)(K >> 6) * t.chunk + t.edge);
+    if (i == 0 || est < tb) {
+      best = i + 1;
+      tb = est;
+    }
+  }
+  return best;
 }
 
 template <int EPI>
 static int launch_f16(int cfg, const f16* x, long ldx, const f16* wp, const float* bias,
                       float alpha, const f16* res, long ldr, f16* y, long ldy, int M, int N,
                       int K, const RowMap& rm, const RopeOut& ro, hipStream_t st) {
-  if (cfg == 0) cfg = default_cfg(M, N, K, EPI == F16_SILU);
-  switch (cfg) {
-    case 1: return launch_cfg<EPI, 4, 1, 2, 8, 2>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 2: return launch_cfg<EPI, 2, 2, 4, 4, 2>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 3: return launch_cfg<EPI, 4, 1, 4, 8, 2>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 4: return launch_cfg<EPI, 4, 1, 4, 8, 3>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 5: return launch_cfg<EPI, 2, 2, 8, 4, 2>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 6: return launch_cfg<EPI, 2, 2, 4, 8, 2>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 7: return launch_cfg<EPI, 2, 2, 4, 4, 3>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 8: return launch_cfg<EPI, 2, 2, 4, 4, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 9: return launch_cfg<EPI, 4, 1, 2, 8, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 10: return launch_cfg<EPI, 4, 1, 2, 4, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 11: return launch_cfg<EPI, 2, 2, 4, 2, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 12: return launch_cfg<EPI, 1, 4, 4, 2, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 13: return launch_cfg<EPI, 1, 4, 4, 4, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 14: return launch_cfg<EPI, 2, 2, 2, 2, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 15: return launch_cfg<EPI, 2, 2, 2, 2, 3, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
-    case 16: return launch_cfg<EPI, 2, 2, 4, 3, 2, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
+  if (cfg == 0) cfg = default_cfg(M, N, K);
+#define F16_CFG(I, ...)                                                                       \
+  case I:                                                                                     \
+    return launch_cfg<EPI, __VA_ARGS__>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, \
+                                        ro, st)
+  switch ((cfg - 1) % 10 + 1) {
+    F16_CFG(1, 4, 2, 2, 4, 2);
+    F16_CFG(2, 4, 2, 2, 3, 2);
+    F16_CFG(3, 4, 2, 2, 2, 3);
+    F16_CFG(4, 4, 2, 1, 3, 3);
+    F16_CFG(5, 4, 2, 1, 2, 4);
+    F16_CFG(6, 2, 2, 2, 1, 5);
+    F16_CFG(7, 2, 2, 1, 2, 5);
+    F16_CFG(8, 2, 2, 1, 1, 8);
+    F16_CFG(9, 4, 2, 1, 2, 2);
+    F16_CFG(10, 2, 4, 1, 1, 2);
     default: return ECD_EINVAL;
   }
+#undef F16_CFG
 }
 
 static int launch_epi(int epi, int cfg, const f16* x, long ldx, const f16* wp, const float* bias,

@@ -452,8 +452,9 @@ int ecd_gemm_f16p_conv_tuned(const void* x, long ldx, const void* wp, const floa
 
 /* ecd_gemm_f16p (epi 0), ecd_gemm_f16p_silu (epi 1, N = 2F, bias/res NULL, alpha 1) or
  * ecd_gemm_f16p_prelu (epi 2, alpha = the slope) with an
- * explicit block tile (cfg 1..16: 128x128, 256x128, 128x256, 128x64, 64x128, 64x256, 64x64 or 128x96 features x rows,
- * 2 to 4 LDS stages; 0 = the library's choice).  Replaces nothing in the reference: the launch-shape knob
+ * explicit block tile (cfg 1..10: 256x256, 256x192, 256x128, 128x192, 128x128, 128x64, 64x128, 64x64
+ * features x rows with one workgroup per CU, then 128x128 and 64x128 with several; 11..16 are 1..6 again;
+ * 0 = the library's choice).  Replaces nothing in the reference: the launch-shape knob
  * of the codec GEMMs, for sweeps. */
 int ecd_gemm_f16p_tuned(const void* x, long ldx, const void* wp, const float* bias, float alpha,
                         const void* res, long ldr, void* y, long ldy, int M, int N, int K,
