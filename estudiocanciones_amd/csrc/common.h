@@ -130,8 +130,11 @@ __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, void* 
 // in M0 (it is not allocatable, and no other instruction of these kernels reads it).
 template <int IMM>
 __device__ __forceinline__ void lds_dma16_at(const void* base, uint32_t off, uint32_t lds) {
+  const uint64_t b = (uint64_t)base;  // uniform; said again, since it may come through a vector register
+  const uint64_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32;
   asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               : : "v"(off), "s"(base), "s"(lds), "i"(IMM) : "memory", "scc");
+               : : "v"(off), "s"(u), "s"(lds), "i"(IMM) : "memory", "scc");
 }
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;

@@ -13,84 +13,16 @@
 // of half h hold row l & 15, k = 64c + 16 (l >> 4) + 8h .. +7 (ecd_pack_f16), so one 16-byte
 // LDS read is an MFMA A fragment.  The activations x are the B operand.
 //
-// Tiling (template): NW = WN x WM waves; wave (wn, wm) owns FT 32-feature tiles and RT 32-row tiles
-// of v_mfma_f32_32x32x16_f16, so a block covers BN = 32 WN FT features x BM = 32 WM RT rows.  (At
-// one wave per SIMD independent 32x32x16 products issued back to back reach 2.14 PFLOP/s on this
-// chip, 16x16x32 ones 1.86.)  K advances in 64-wide chunks that go straight from global memory into
-// an NS-stage LDS ring (LDS DMA, no register staging); x rows are stored with their 16-byte pieces
-// XOR-swizzled by row (piece p of row r at position p ^ ((r >> 1) & 7)), so that the 16 rows that a
-// ds_read_b128 serves at a time lie in distinct banks (no conflicts counted).
-//
-// What bounds it: a CU takes about 57 bytes per clock through its vector memory path (measured, L2
-// hits), so a block tile needs a high ratio of products to bytes: 128 x 128 needs 575 clocks of
-// loads for 512 of MFMA per chunk, 256 x 256 1150 for 2048.  Loads that miss L2 take 1 to 2 us, so a
-// small tile needs many chunks in flight: NS is what the LDS holds.  Fragments are read half a chunk
-// ahead, interleaved with the products; each DMA takes three instructions (computing every address
-// on the scalar unit took twelve, and the issue slots of a third of the loop).  The output goes through
-// LDS (see the epilogue).  us before -> now, M = 1488 (N, K): (4608, 1536) 31.8 -> 25.7, (8192, 1536)
-// 56.3 -> 41.5, (1536, 1536) 16.6 -> 14.1, (1536, 4096) 36.3 -> 28.2, (9216, 3072) 102 -> 80,
-// (16384, 3072) 182 -> 145, (3072, 8192) 111 -> 84; M = 187: (4608, 1536) 19.8 -> 9.9,
-// (1536, 4096) 26.1 -> 14.4, (3072, 8192) 99.7 -> 36.8; 8192^3 0.90 -> 1.21 PFLOP/s.
+// Tiles and main loop: gemm_core.h.
 //
 // Block order is XCD-aware: the row blocks that share a weight tile get block ids equal modulo 8,
 // so they run on one XCD and share its L2 (feature blocks in whole groups of 8; the grid has
 // exactly one workgroup per output tile, so narrow outputs launch no empty workgroups).
-#include "common.h"
+#include "gemm_core.h"
 
 namespace ecd {
 
 enum { F16_STORE = 0, F16_SILU = 1, F16_PRELU = 2, F16_ROPE = 3 };
-
-// wait until at most N vector-memory operations of this wave are outstanding and its LDS
-// operations are done (lgkmcnt 0)
-template <int N>
-__device__ __forceinline__ void wait_vm_lgkm0() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
-}
-
-// wait for this wave's DMA of one chunk while the `later` chunks issued after it (uniform,
-// 0 .. MAXL) stay in flight; PER instructions per chunk; LGKM: also drain LDS operations
-template <int PER, int MAXL, bool LGKM>
-__device__ __forceinline__ void wait_chunk(int later) {
-  if constexpr (MAXL >= 1) {
-    if (later < MAXL) {
-      wait_chunk<PER, MAXL - 1, LGKM>(later);
-      return;
-    }
-  }
-  if constexpr (LGKM) wait_vm_lgkm0<MAXL * PER>(); else wait_vm<MAXL * PER>();
-}
-
-template <int I>
-struct IC {
-  static constexpr int value = I;
-};
-// f(IC<B>{}), .., f(IC<E - 1>{})
-template <int B, int E, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (B < E) {
-    f(IC<B>{});
-    static_for<B + 1, E>(f);
-  }
-}
-
-// The fragments of half a 64-wide chunk, two k-steps of v_mfma_f32_32x32x16_f16: lane l holds
-// feature (or row) l & 31 of a 32-wide tile, k = 16 s + 8 (l >> 5) .. + 7 of step s.
-template <int FT, int RT>
-struct Frags {
-  f16x8 w[2][FT], x[2][RT];
-};
-
-// Row layouts of a convolution as a GEMM over implicit tap columns (the waveform decoder):
-// row m = b * T + t of the GEMM.  With k > 0, x is time-major with xpad zero rows before each
-// sequence and row m's K index j * C + c (C = 64 cpt) reads x row b (T + xpad) + xpad + t + off[j]
-// (the tap offsets move the chunk's DMA base; the pad rows supply the zeros of the padding).
-// With ypad >= 0, y and res rows are b (T + ypad) + ypad + t.  T = 0: plain rows throughout.
-struct RowMap {
-  int T, xpad, ypad, cpt, k, rep;
-  int off[8];
-};
 
 // Output of the q | k | v projection with RoPE (F16_ROPE): features [0, D) are q, [D, 2D) k,
 // [2D, 3D) v, D = H * HD, rows m = b * T + t.  q and k pairs (2i, 2i + 1) are rotated by
@@ -101,300 +33,125 @@ struct RopeOut {
   int T, H, HD;
 };
 
-__device__ __forceinline__ long seq_row(int m, int T, int pad) {
-  const int b = m / T;
-  return (long)b * (T + pad) + pad + (m - b * T);
-}
-
-// piece p of x row r lies at position p ^ x_swz(r) of its 128 bytes
-__device__ __forceinline__ int x_swz(int r) { return (r >> 1) & 7; }
-
 template <int EPI, int WN, int WM, int FT, int RT, int NS>
 __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
     const f16* __restrict__ x, long ldx, const f16* __restrict__ wp,
     const float* __restrict__ bias, float alpha, const f16* res, long ldr,
     f16* y, long ldy, int M, int N, int K, int nfb, int nmb, RowMap rm,
     RopeOut ro) {
-  constexpr int NW = WN * WM;           // waves
-  constexpr int BN = 32 * WN * FT;      // features per block
-  constexpr int BM = 32 * WM * RT;      // rows per block
-  constexpr int WI = BN / 8 / NW;       // weight DMA instructions per wave per chunk (1 KB each)
-  constexpr int XI = BM / 8 / NW;       // x DMA instructions per wave per chunk (8 rows each)
-  constexpr int PER_CHUNK = WI + XI;
-  static_assert(WI * 8 * NW == BN && XI * 8 * NW == BM, "whole DMA instructions per wave");
-  static_assert(NS >= 2 && PER_CHUNK * (NS - 1) < 64, "vmcnt range");
-  constexpr int LW = BN * 64, LX = BM * 64, STG = LW + LX;  // halfs per stage
-  __shared__ __align__(16) f16 lds[NS * STG];
-
-  // feature blocks in full groups of 8 share XCDs with their row blocks; the remaining
-  // nfb % 8 feature blocks (all of them when nfb < 8) are laid out row-major after them
-  const int b = blockIdx.x;
-  const int full = nfb & ~7;
+  using G = GemmTile<false, false, WN, WM, FT, RT, NS>;
+  __shared__ __align__(16) f16 lds[G::LDS_HALFS];
   int fb, mb;
-  if (b < full * nmb) {
-    const int grp8 = b / (8 * nmb);
-    const int rem = b - grp8 * 8 * nmb;
-    mb = rem >> 3;
-    fb = grp8 * 8 + (rem & 7);
-  } else {
-    const int rem = b - full * nmb;
-    const int tw = nfb - full;
-    mb = rem / tw;
-    fb = full + (rem - mb * tw);
-  }
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wn = wv % WN, wm = wv / WN;
-  const int n0 = fb * BN;
-  const int m0 = mb * BM;
-  const int nch = K >> 6;
-  const int ntiles = (N + 15) >> 4;
-  const long tile_bytes = (long)nch * 2048;
-
-  // DMA sources: weight instruction j of this wave is tile t = i >> 1, half h = i & 1 with
-  // i = wv + NW j (tiles past N re-read the last tile; their results are never stored); x
-  // instruction j covers rows 8 i .. 8 i + 7, i = wv + NW j (rows past M re-read row M - 1).
-  // Every address is a uniform base, advanced per chunk, plus a per-lane offset.
-  const int t0 = min(n0 / 16, ntiles - 1);
-  const char* wb = (const char*)wp + (long)t0 * tile_bytes;
-  uint32_t woff[WI];
-#pragma unroll
-  for (int j = 0; j < WI; ++j) {
-    const int i = wv + NW * j;
-    woff[j] = (uint32_t)((min(n0 / 16 + (i >> 1), ntiles - 1) - t0) * tile_bytes) + 1024 * (i & 1) + 16 * lane;
-  }
-  // with a 2x row-repeat (rm.rep == 2) output step t reads source row (t + o) >> 1 for tap o:
-  // (t >> 1) + (o >> 1) for even o, ((t + 1) >> 1) + (o >> 1) for odd o -- two lane rows
-  uint32_t xoff[XI], xoff1[XI];
-#pragma unroll
-  for (int j = 0; j < XI; ++j) {
-    const int i = wv + NW * j;
-    const int xpiece = (lane & 7) ^ x_swz(8 * i + (lane >> 3));
-    const int row = min(m0 + 8 * i + (lane >> 3), M - 1);
-    long xr = row, xr1 = row;
-    if (rm.k && rm.rep == 2) {
-      const int b = row / rm.T, t = row - b * rm.T;
-      const long base = (long)b * (rm.T / 2 + rm.xpad) + rm.xpad;
-      xr = base + (t >> 1);
-      xr1 = base + ((t + 1) >> 1);
-    } else if (rm.k) {
-      xr = xr1 = seq_row(row, rm.T, rm.xpad);
-    }
-    xoff[j] = (uint32_t)(xr * ldx * 2 + 16 * xpiece);
-    xoff1[j] = (uint32_t)(xr1 * ldx * 2 + 16 * xpiece);
-  }
-  // x base of the next chunk to load: plain K offset 64 c, or tap j = c / cpt shifted by off[j]
-  // rows (by off[j] >> 1 with a 2x row-repeat, odd taps reading the second set of lane rows)
-  const f16* xb = x;
-  int tap = 0, tc = 0;
-  bool odd = false;
-  auto set_tap = [&]() {
-    const int o = rm.off[tap];
-    odd = rm.rep == 2 && (o & 1);
-    xb = x + (long)(rm.rep == 2 ? (o >> 1) : o) * ldx;
-  };
-  if (rm.k) set_tap();
-  auto next_chunk = [&]() {
-    xb += 64;
-    wb += 2048;
-    if (rm.k && ++tc == rm.cpt) {
-      tc = 0;
-      ++tap;
-      if (tap < rm.k) set_tap();
-    }
-  };
-  // DMA instruction J of the next chunk into the stage at LDS byte address `sa` (this wave's first
-  // KB of it): weights first, then x rows
-  auto dma = [&](auto J, uint32_t sa) {
-    constexpr int j = decltype(J)::value;
-    if constexpr (j < WI)
-      lds_dma16_at<NW * j * 1024>(wb, woff[j], sa);
-    else
-      lds_dma16_at<LW * 2 + NW * (j - WI) * 1024>(xb, odd ? xoff1[j - WI] : xoff[j - WI], sa);
-  };
-  const uint32_t lds0 = lds_addr(lds) + wv * 1024;
-
-  f32x16 acc[FT][RT];
-  static_for<0, FT * RT>([&](auto I) {
-    acc[I.value / RT][I.value % RT] = (f32x16)(0.f);
-  });
-
-  // fragment addresses within a stage (halfs): a 32-feature tile is two packed 16-row tiles, octet
-  // o = 2 s + (lane >> 5) of k-step s lies in half o & 1 = lane >> 5 at 16-byte unit 16 s + row
-  const int wfo = (wn * FT * 2 + ((lane >> 4) & 1)) * 1024 + (lane >> 5) * 512 + (lane & 15) * 8;
-  int xfo[4];
-  static_for<0, 4>([&](auto S) {
-    xfo[S.value] = LW + (wm * RT * 32 + (lane & 31)) * 64 +
-                   8 * ((2 * S.value + (lane >> 5)) ^ x_swz(lane & 31));
-  });
-
-  // read I of a half chunk's fragments (k-steps 2 H and 2 H + 1), k-step by k-step
-  constexpr int NM = 2 * FT * RT, NR = 2 * (FT + RT);
-  auto read1 = [&](auto I, auto H, const f16* base, Frags<FT, RT>& f) {
-    constexpr int s = decltype(I)::value / (FT + RT), i = decltype(I)::value % (FT + RT);
-    constexpr int ks = 2 * decltype(H)::value + s;
-    if constexpr (i < FT)
-      f.w[s][i] = *(const f16x8*)(base + wfo + 128 * ks + i * 2048);
-    else
-      f.x[s][i - FT] = *(const f16x8*)(base + xfo[ks] + (i - FT) * 2048);
-  };
-  // the products of a half chunk, interleaved with the reads of the next half chunk's fragments
-  // (in the first half of the products, so that they have landed at its end) and, with LOAD, the
-  // loads of a later chunk
-  auto half = [&](const Frags<FT, RT>& f, auto H, const f16* base, Frags<FT, RT>& nf, auto LOAD,
-                  uint32_t sa) {
-    constexpr int RH = NM / 2;
-    static_for<0, NM>([&](auto I) {
-      constexpr int m = decltype(I)::value, s = m / (FT * RT), ft = m % (FT * RT) / RT, rt = m % RT;
-      acc[ft][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.w[s][ft], f.x[s][rt], acc[ft][rt], 0, 0, 0);
-      if constexpr (decltype(LOAD)::value)
-        static_for<m * PER_CHUNK / NM, (m + 1) * PER_CHUNK / NM>([&](auto J) { dma(J, sa); });
-      if constexpr (m < RH)
-        static_for<m * NR / RH, (m + 1) * NR / RH>([&](auto J) { read1(J, H, base, nf); });
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  };
-
-  for (int s = 0; s < NS; ++s)
-    if (s < nch) {
-      static_for<0, PER_CHUNK>([&](auto J) { dma(J, lds0 + s * (STG * 2)); });
-      next_chunk();
-    }
-  wait_chunk<PER_CHUNK, NS - 1, false>(min(NS - 1, nch - 1));
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  Frags<FT, RT> fa, fc;
-  static_for<0, NR>([&](auto I) { read1(I, IC<0>{}, lds, fa); });
-
-  // Chunk c: its first half while its second half is read; then, with chunk c + 1 landed for this
-  // wave (later ones may fly) and its own reads of chunk c done, a barrier that publishes the one and
-  // frees the stage of the other; then the second half while chunk c + 1's first half is read and
-  // chunk c + NS loaded into the stage left free.
-  int c = 0, st = 0;  // st: stage of chunk c
-  for (; c < nch - NS; ++c) {
-    half(fa, IC<1>{}, lds + st * STG, fc, IC<0>{}, 0);
-    wait_vm_lgkm0<(NS - 2) * PER_CHUNK>();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    const int sn = st + 1 == NS ? 0 : st + 1;
-    half(fc, IC<0>{}, lds + sn * STG, fa, IC<1>{}, lds0 + st * (STG * 2));
-    next_chunk();
-    st = sn;
-  }
-  for (; c < nch; ++c) {
-    half(fa, IC<1>{}, lds + st * STG, fc, IC<0>{}, 0);
-    if (c + 1 < nch) {
-      wait_chunk<PER_CHUNK, NS - 2, true>(min(NS - 2, nch - 2 - c));
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-    }
-    // (behind the last chunk the reads return a stage's old contents, never used)
-    const int sn = st + 1 == NS ? 0 : st + 1;
-    half(fc, IC<0>{}, lds + sn * STG, fa, IC<0>{}, 0);
-    st = sn;
-  }
-
-  // Epilogue.  A lane holds features 8 g + 4 (lane >> 5) .. + 3 (g < 4) of row lane & 31 of each of
-  // its tiles.  The rounded sums go through LDS (the stages are free once every wave has read its last
-  // fragments), so that a short loop finishes them in 16-byte pieces of consecutive features and
-  // writes whole row segments.  Unrolled over the accumulators, with 8-byte stores to 32 rows per
-  // instruction, the same work took about 1.1 us per 32 x 32 tile of a wave, most of it instruction
-  // fetch (the code runs once per workgroup).
-  constexpr int PR = BN / 8;                       // 16-byte pieces per row
-  constexpr int SM = PR < 16 ? PR - 1 : 15;
-  auto piece = [](int r, int p) { return (r * PR + (p ^ (r & SM))) * 8; };  // in halfs
-  static_assert(NS * STG >= BM * BN, "the output tile fits the stages");
-  __syncthreads();
-  static_for<0, 4 * FT>([&](auto I) {
-    constexpr int ft = decltype(I)::value >> 2, g = decltype(I)::value & 3;
-    const int nl = (wn * FT + ft) * 32 + 8 * g + 4 * (lane >> 5);
-    f32x4 bv = (f32x4){0.f, 0.f, 0.f, 0.f};
-    if (bias) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) bv[r] = bias[min(n0 + nl + r, N - 1)];
-    }
-    static_for<0, RT>([&](auto R) {
-      constexpr int rt = decltype(R)::value;
-      const int r = (wm * RT + rt) * 32 + (lane & 31);
-      f16x4 yv;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) yv[j] = (f16)(acc[ft][rt][4 * g + j] + bv[j]);
-      *(f16x4*)(lds + piece(r, nl >> 3) + (nl & 4)) = yv;
-    });
-  });
-  __syncthreads();
+  G::block(nfb, nmb, fb, mb);
+  const int n0 = fb * G::BN, m0 = mb * G::BM;
+  G::run(lds, x, ldx, wp, nullptr, bias, M, N, K, n0, m0, rm);
   // 16-byte rows of y (and res) take one store per piece
   const bool vec = ((ldy & 7) == 0) && (((uintptr_t)y & 15) == 0) &&
                    (!res || (((ldr & 7) == 0) && (((uintptr_t)res & 15) == 0)));
+  constexpr int U = G::U;
+  const int p = threadIdx.x % G::PR, nb = n0 + 8 * p;
+  if (nb >= N) return;
+  const bool full = nb + 7 < N;
+  // F16_ROPE (HD % 4 == 0): sections (q, k, v), heads and offsets of the piece's two groups of 4 features
+  const int D = ro.H * ro.HD;
+  int sec[2], hh[2], hd[2];
+  if constexpr (EPI == F16_ROPE) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int n = nb + 4 * q;
+      sec[q] = n >= 2 * D ? 2 : (n >= D ? 1 : 0);
+      hh[q] = (n - sec[q] * D) / ro.HD;
+      hd[q] = n - sec[q] * D - hh[q] * ro.HD;
+    }
+  }
 #pragma unroll 1
-  for (int i = tid; i < BM * PR; i += 64 * NW) {
-    const int r = i / PR, p = i - r * PR;
-    const int mm = m0 + r, nb = n0 + 8 * p;
-    if (mm >= M || nb >= N) continue;
-    f16x8 v = *(const f16x8*)(lds + piece(r, p));
+  for (int r0 = threadIdx.x / G::PR; r0 < G::BM; r0 += G::RS * U) {
+    if (m0 + r0 >= M) break;
+    f16x8 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = *(const f16x8*)(lds + G::piece(r0 + G::RS * u, p));
     if constexpr (EPI == F16_STORE || EPI == F16_PRELU) {
-      const long m = rm.ypad >= 0 ? seq_row(mm, rm.T, rm.ypad) : mm;
-      if constexpr (EPI == F16_PRELU) {  // alpha: the slope
+      long m[U];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if ((float)v[j] < 0.f) v[j] = (f16)((float)v[j] * alpha);
-      } else if (alpha != 1.0f) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (f16)((float)v[j] * alpha);
+      for (int u = 0; u < U; ++u) {
+        const int mm = min(m0 + r0 + G::RS * u, M - 1);
+        m[u] = rm.ypad >= 0 ? seq_row(mm, rm.T, rm.ypad) : mm;
       }
-      if (vec && nb + 7 < N) {
-        if (res) v = v + *(const f16x8*)(res + m * ldr + nb);
-        *(f16x8*)(y + m * ldy + nb) = v;
-      } else {
-        for (int j = 0; j < 8 && nb + j < N; ++j) {
-          f16 o = v[0];
-          if (res) o = o + res[m * ldr + nb + j];
-          y[m * ldy + nb + j] = o;
-          v = __builtin_shufflevector(v, v, 1, 2, 3, 4, 5, 6, 7, 0);
+      f16x8 rv[U];
+      if (res && vec && full) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) rv[u] = *(const f16x8*)(res + m[u] * ldr + nb);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (m0 + r0 + G::RS * u >= M) break;
+        if constexpr (EPI == F16_PRELU) {  // alpha: the slope
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if ((float)v[u][j] < 0.f) v[u][j] = (f16)((float)v[u][j] * alpha);
+        } else if (alpha != 1.0f) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[u][j] = (f16)((float)v[u][j] * alpha);
+        }
+        if (vec && full) {
+          *(f16x8*)(y + m[u] * ldy + nb) = res ? v[u] + rv[u] : v[u];
+        } else {
+          for (int j = 0; j < 8 && nb + j < N; ++j) {
+            f16 o = v[u][0];
+            if (res) o = o + res[m[u] * ldr + nb + j];
+            y[m[u] * ldy + nb + j] = o;
+            v[u] = __builtin_shufflevector(v[u], v[u], 1, 2, 3, 4, 5, 6, 7, 0);
+          }
         }
       }
     } else if constexpr (EPI == F16_ROPE) {
-      // sections q, k, v; 4 features never straddle a head (HD % 4 == 0)
-      const int D = ro.H * ro.HD;
-      const int rb = mm / ro.T, t = mm - rb * ro.T;
+      int rb[U], t[U];
+      f16x4 cs[U][2];  // pairs d / 2, d / 2 + 1
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int n = nb + 4 * q;
-        if (n >= N) break;
-        const int sec = n >= 2 * D ? 2 : (n >= D ? 1 : 0);
-        const int hc = n - sec * D, hh = hc / ro.HD, d = hc - hh * ro.HD;
-        f16x4 o = q ? __builtin_shufflevector(v, v, 4, 5, 6, 7) : __builtin_shufflevector(v, v, 0, 1, 2, 3);
-        if (sec < 2) {
-          const f16x4 cs = *(const f16x4*)(ro.tab + (long)t * ro.HD + d);  // pairs d/2, d/2 + 1
-          f16 o0, o1, o2, o3;
-          rope_pair_f16((float)o[0], (float)o[1], (float)cs[0], (float)cs[1], o0, o1);
-          rope_pair_f16((float)o[2], (float)o[3], (float)cs[2], (float)cs[3], o2, o3);
-          o = (f16x4){o0, o1, o2, o3};
+      for (int u = 0; u < U; ++u) {
+        const int mm = min(m0 + r0 + G::RS * u, M - 1);
+        rb[u] = mm / ro.T;
+        t[u] = mm - rb[u] * ro.T;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) cs[u][q] = *(const f16x4*)(ro.tab + (long)t[u] * ro.HD + hd[q]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int mm = m0 + r0 + G::RS * u;
+        if (mm >= M) break;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          if (nb + 4 * q >= N) break;
+          f16x4 o = q ? __builtin_shufflevector(v[u], v[u], 4, 5, 6, 7)
+                      : __builtin_shufflevector(v[u], v[u], 0, 1, 2, 3);
+          if (sec[q] < 2) {
+            const f16x4 c = cs[u][q];
+            f16 o0, o1, o2, o3;
+            rope_pair_f16((float)o[0], (float)o[1], (float)c[0], (float)c[1], o0, o1);
+            rope_pair_f16((float)o[2], (float)o[3], (float)c[2], (float)c[3], o2, o3);
+            o = (f16x4){o0, o1, o2, o3};
+          }
+          f16* dst = sec[q] == 0 ? ro.q + (long)mm * D + hh[q] * ro.HD + hd[q]
+                                 : (sec[q] == 1 ? ro.k : ro.v) +
+                                       (((long)rb[u] * ro.H + hh[q]) * ro.T + t[u]) * ro.HD + hd[q];
+          *(f16x4*)dst = o;
         }
-        f16* dst = sec == 0 ? ro.q + (long)mm * D + hc
-                            : (sec == 1 ? ro.k : ro.v) + (((long)rb * ro.H + hh) * ro.T + t) * ro.HD + d;
-        *(f16x4*)dst = o;
       }
     } else {  // pairs (a_j, b_j) with j = nb / 2 ..; N even
-      f16x2 o[4];
+      const bool v8 = full && ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float a = (float)v[2 * q];
-        const f16 s = (f16)(a / (1.0f + expf(-a))) * v[2 * q + 1];
-        o[q >> 1][q & 1] = s;
-      }
-      f16* dst = y + (long)mm * ldy + (nb >> 1);
-      if (nb + 7 < N && ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0)) {
-        *(f16x4*)dst = (f16x4){o[0].x, o[0].y, o[1].x, o[1].y};
-      } else {
+      for (int u = 0; u < U; ++u) {
+        const int mm = m0 + r0 + G::RS * u;
+        if (mm >= M) break;
+        const f16x4 o = silu_mul4(v[u]);
+        f16* dst = y + (long)mm * ldy + (nb >> 1);
+        if (v8) {
+          *(f16x4*)dst = o;
+        } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (nb + 2 * q < N) dst[q] = o[q >> 1][q & 1];
+          for (int q = 0; q < 4; ++q)
+            if (nb + 2 * q < N) dst[q] = o[q];
+        }
       }
     }
   }
@@ -438,20 +195,22 @@ static int launch_cfg(const f16* x, long ldx, const f16* wp, const float* bias, 
 }
 
 // The tiles (features x rows, LDS stages).  1 to 8 leave room for one workgroup per CU: a launch takes
-// ceil(blocks / 256) rounds, a round about K / 64 chunk times plus a fill and an epilogue; both in ns,
-// measured over K = 1536 .. 8192 with 100 to 256 workgroups.
+// ceil(blocks / 256) rounds, a round about K / 64 chunk times plus a fill and an epilogue.  In ns,
+// measured over K = 1536 .. 8192; a chunk takes longer when all CUs load at once (`full`: 256 workgroups)
+// than with at most LIGHT of them (`light`).
 struct Tile {
-  int bn, bm, chunk, edge;
+  int bn, bm, light, full, edge;
 };
+constexpr int LIGHT = 144;
 constexpr Tile TILES[8] = {
-    {256, 256, 1550, 4500},  // 1: 8 waves of 64 x 128, 2 stages
-    {256, 192, 1450, 3500},  // 2: 8 waves of 64 x 96, 2 stages
-    {256, 128, 850, 2500},   // 3: 8 waves of 64 x 64, 3 stages
-    {128, 192, 620, 3000},   // 4: 8 waves of 32 x 96, 3 stages
-    {128, 128, 440, 1200},   // 5: 8 waves of 32 x 64, 4 stages
-    {128, 64, 300, 800},     // 6: 4 waves of 64 x 32, 5 stages
-    {64, 128, 300, 800},     // 7: 4 waves of 32 x 64, 5 stages
-    {64, 64, 220, 600},      // 8: 4 waves of 32 x 32, 8 stages
+    {256, 256, 1300, 1550, 5000},  // 1: 8 waves of 64 x 128, 2 stages
+    {256, 192, 1190, 1450, 3500},  // 2: 8 waves of 64 x 96, 2 stages
+    {256, 128, 750, 870, 2500},    // 3: 8 waves of 64 x 64, 3 stages
+    {128, 192, 660, 800, 3000},    // 4: 8 waves of 32 x 96, 3 stages
+    {128, 128, 440, 670, 1200},    // 5: 8 waves of 32 x 64, 4 stages
+    {128, 64, 280, 420, 800},      // 6: 4 waves of 64 x 32, 5 stages
+    {64, 128, 280, 420, 800},      // 7: 4 waves of 32 x 64, 5 stages
+    {64, 64, 200, 260, 600},       // 8: 4 waves of 32 x 32, 8 stages
 };
 // 9: 128 x 128, 8 waves, 2 stages; 10: 64 x 128, 8 waves, 2 stages: several workgroups per CU, for the
 // waveform decoder's convolutions of at most 128 channels over many rows, whose few chunks leave the
@@ -469,7 +228,9 @@ static int default_cfg(int M, int N, int K) {
   for (int i = 0; i < 8; ++i) {
     const Tile& t = TILES[i];
     const long blocks = (long)((N + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
-    const long est = (blocks + 255) / 256 * ((long)(K >> 6) * t.chunk + t.edge);
+    const long load = blocks <= LIGHT ? 0 : (blocks >= 256 ? 256 - LIGHT : blocks - LIGHT);
+    const long chunk = t.light + (t.full - t.light) * load / (256 - LIGHT);
+    const long est = (blocks + 255) / 256 * ((K >> 6) * chunk + t.edge);
     if (i == 0 || est < tb) {
       best = i + 1;
       tb = est;

@@ -14,26 +14,17 @@
 // layout int8_mm receives, app/kernels.py:40-49): the DMA lands them in LDS in the same lane
 // order, so everything after the load is shared.
 //
-// Tiling: a block computes 128 output features x 128 rows with 4 waves; wave w owns features
-// 32 w .. 32 w + 31 for all 128 rows = 2 x 8 tiles of v_mfma_f32_16x16x32_f16 (weights = A
-// operand, x = B operand), so each weight fragment is dequantised by one wave only (the
-// dequantisation is the kernel's largest VALU cost).  K advances in 64-wide chunks that go straight from global memory into two LDS
-// stages (global_load_lds_dwordx4: each wave instruction writes 1 KB of LDS in lane order): the
-// next chunk is in flight while one is multiplied, no registers stage the data, and 48 KB of
-// LDS per block leave room for three blocks per CU.
-// Weights arrive as packed 1 KB tiles; the 16-byte pieces of each x row (128 bytes per chunk)
-// are XOR-swizzled by row (piece p of row r at position p ^ (r & 7)), which the loads produce
-// by choosing each lane's source and which spreads the fragment reads over the banks.  Each
-// 16-byte weight fragment is dequantised once and used by 8 row tiles; each x fragment is used
-// by 2 feature tiles.
-//
-// The kernel orders the DMA itself: at the top of step c each thread waits for its own loads of
-// chunk c (vmcnt 0), a barrier makes the chunk of every wave visible and frees the stage read
-// in step c - 1, and only then are chunk c + 1's loads issued into that stage.
+// Tiles and main loop: gemm_core.h.  At few rows the former kernel (128 x 128 tiles, two stages) left
+// most CUs idle and waited 0.6 us for each 64-wide chunk; deeper rings and smaller tiles took, in us
+// (M = 154; N, K): (5120, 3072) 36.5 -> 17.1, (3072, 3072) 30.4 -> 16.4, (16384, 3072) 39.4 -> 27.7,
+// (3072, 8192) 91.6 -> 35.7.  At 2048 rows it is bound
+// by the products, the conversion and the LDS reads together: (3072, 3072) 46.6 -> 42.5,
+// (16384, 3072) 197 -> 192, (3072, 8192) 110 -> 102 (1.01 PFLOP/s); at 4096 rows (16384, 3072) 442 -> 397,
+// but (5120, 3072) 131 -> 138 and (3072, 8192) 202 -> 214, where 256 x 128 tiles make 1.5 rounds.
 //
 // Block order is XCD-aware: the row blocks that share a weight tile get block ids that are
 // equal modulo 8, so they run on one XCD and re-read the tile from its L2.
-#include "common.h"
+#include "gemm_core.h"
 
 namespace ecd {
 
@@ -50,184 +41,187 @@ struct RopeOut {
   int S, Hq, Hk, L, HD;
 };
 
-constexpr int GT_N = 128;   // output features per block
-constexpr int GT_M = 128;   // rows per block
-constexpr int GT_NS = 2;    // LDS stages
-
-template <int EPI, bool RM>
-__global__ __launch_bounds__(256) void gemm_i8p_kernel(
+template <int EPI, bool RM, int WN, int WM, int FT, int RT, int NS>
+__global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_kernel(
     const f16* __restrict__ x, long ldx, const int8_t* __restrict__ wp,
-    const f16* __restrict__ s, const f16* __restrict__ res, long ldr, f16* __restrict__ y, long ldy, int M, int N, int K,
-    int nfb, int nmb, RopeOut ro) {
-  constexpr int WB = 1024;  // bytes of one (tile, chunk) of packed weights
-  __shared__ __align__(16) int8_t lw[GT_NS][8 * WB];
-  __shared__ __align__(16) f16 lx[GT_NS][GT_M * 64];
-
-  // XCD-aware block order: blocks b and b + 8 run on the same XCD.  Feature block fb and row
-  // block mb map to b = (fb / 8) * (8 * nmb) + mb * 8 + fb % 8.
-  const int b = blockIdx.x;
-  const int grp8 = b / (8 * nmb);
-  const int rem = b - grp8 * 8 * nmb;
-  const int mb = rem >> 3;
-  const int fb = grp8 * 8 + (rem & 7);
-  if (fb >= nfb) return;  // padding blocks of the last group of 8 (uniform per block)
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = fb * GT_N;
-  const int m0 = mb * GT_M;
-  const int nch = K >> 6;
-  const int ntiles = (N + 15) >> 4;
-
-  // sources of this thread's loads: weight tiles wv and wv + 4 (16 bytes of each 1 KB chunk);
-  // x rows 8 (4 wv + i) + (lane >> 3), swizzled piece (lane & 7) ^ (lane >> 3).  Rows past M
-  // read row M - 1 and tiles past N the last tile (their results are never stored), so every
-  // thread issues the same number of loads.
-  // The addresses are a wave-uniform base (SGPRs, advanced per chunk by scalar adds) plus a
-  // per-lane byte offset fixed for the whole loop (the host keeps the x buffer below 2 GiB).
-  const int t0 = min(n0 / 16 + wv, ntiles - 1), t1 = min(n0 / 16 + 4 + wv, ntiles - 1);
-  const int8_t* wbase0 = wp + (RM ? (long)t0 * 16 * K : (long)t0 * nch * WB);
-  const int8_t* wbase1 = wp + (RM ? (long)t1 * 16 * K : (long)t1 * nch * WB);
-  // row-major: row 16 t + (lane & 15) (the last row for rows past N), bytes 16 (lane >> 4) of
-  // each 64-byte chunk; the per-lane offsets stay below 16 K bytes
-  const uint32_t woff0 = RM ? (uint32_t)((min(16 * t0 + (lane & 15), N - 1) - 16 * t0) * K +
-                                         16 * (lane >> 4))
-                            : 16u * lane;
-  const uint32_t woff1 = RM ? (uint32_t)((min(16 * t1 + (lane & 15), N - 1) - 16 * t1) * K +
-                                         16 * (lane >> 4))
-                            : 16u * lane;
-  constexpr long WSTEP = RM ? 64 : WB;  // bytes between consecutive chunks of a tile
-  const int xpiece = (lane & 7) ^ (lane >> 3);
-  uint32_t xoff[4];
+    const f16* __restrict__ s, const f16* __restrict__ res, long ldr, f16* __restrict__ y, long ldy,
+    int M, int N, int K, int nfb, int nmb, RopeOut ro) {
+  using G = GemmTile<true, RM, WN, WM, FT, RT, NS>;
+  __shared__ __align__(16) f16 lds[G::LDS_HALFS];
+  int fb, mb;
+  G::block(nfb, nmb, fb, mb);
+  const int n0 = fb * G::BN, m0 = mb * G::BM;
+  const RowMap rm = {0, 0, -1, 0, 0, 1, {0, 0, 0, 0, 0, 0, 0, 0}};  // plain rows
+  G::run(lds, x, ldx, wp, s, nullptr, M, N, K, n0, m0, rm);
+  const bool vec = ((ldy & 7) == 0) && (((uintptr_t)y & 15) == 0) &&
+                   (!res || (((ldr & 7) == 0) && (((uintptr_t)res & 15) == 0)));
+  constexpr int U = G::U;
+  const int p = threadIdx.x % G::PR, nb = n0 + 8 * p;
+  if (nb >= N) return;
+  const bool full = nb + 7 < N;
+  // GEPI_ROPE (HD % 4 == 0): heads and offsets of the piece's two groups of 4 features
+  int hh[2], hd[2];
+  if constexpr (EPI == GEPI_ROPE) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    xoff[i] = (uint32_t)((long)min(m0 + 8 * (4 * wv + i) + (lane >> 3), M - 1) * ldx * 2 +
-                         16 * xpiece);
-  auto issue = [&](int c, int st) {
-    lds_dma16(wbase0 + (long)c * WSTEP, woff0, &lw[st][wv * WB]);
-    lds_dma16(wbase1 + (long)c * WSTEP, woff1, &lw[st][(4 + wv) * WB]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      lds_dma16(x + (long)c * 64, xoff[i], &lx[st][8 * (4 * wv + i) * 64]);
-  };
-
-  // per-lane dequantisation scales of the 2 feature tiles (row lane & 15 of each)
-  f16 sc[2];
-#pragma unroll
-  for (int ft = 0; ft < 2; ++ft) sc[ft] = s[min(n0 + (wv * 2 + ft) * 16 + (lane & 15), N - 1)];
-
-  f32x4 acc[2][8];
-#pragma unroll
-  for (int ft = 0; ft < 2; ++ft)
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt) acc[ft][rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  issue(0, 0);
-  const int sw = lane & 7;  // swizzle of the rows this lane reads (row & 7 == lane & 7)
-  for (int c = 0; c < nch; ++c) {
-    wait_vm0();  // this thread's loads of chunk c have landed in LDS
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();  // chunk c in LDS for every wave; stage of c - 1 free
-    asm volatile("" ::: "memory");
-    if (c + 1 < nch) issue(c + 1, (c + 1) & 1);
-    const int st = c & 1;
-    f16x8 wa[2], wb[2];
-#pragma unroll
-    for (int ft = 0; ft < 2; ++ft) {
-      const u32x4 raw = *(const u32x4*)(&lw[st][(wv * 2 + ft) * 1024 + 16 * lane]);
-      i8x16_to_f16(raw, wa[ft], wb[ft]);
-      wa[ft] = wa[ft] * sc[ft];
-      wb[ft] = wb[ft] * sc[ft];
-    }
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt) {
-      const f16* xr = &lx[st][(rt * 16 + (lane & 15)) * 64];
-      const int p0 = 2 * (lane >> 4);
-      const f16x8 fa = *(const f16x8*)(xr + 8 * (p0 ^ sw));
-      const f16x8 fb2 = *(const f16x8*)(xr + 8 * ((p0 + 1) ^ sw));
-#pragma unroll
-      for (int ft = 0; ft < 2; ++ft) {
-        acc[ft][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[ft], fa, acc[ft][rt], 0, 0, 0);
-        acc[ft][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb[ft], fb2, acc[ft][rt], 0, 0, 0);
-      }
+    for (int q = 0; q < 2; ++q) {
+      hh[q] = (nb + 4 * q) / ro.HD;
+      hd[q] = nb + 4 * q - hh[q] * ro.HD;
     }
   }
-
-  // epilogue: lane holds features nb + r (r < 4) of row m for every (ft, rt)
-  const bool vec = ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0) &&
-                   (!res || (((ldr & 3) == 0) && (((uintptr_t)res & 7) == 0)));
+#pragma unroll 1
+  for (int r0 = threadIdx.x / G::PR; r0 < G::BM; r0 += G::RS * U) {
+    if (m0 + r0 >= M) break;
+    f16x8 v[U];
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt) {
-    const int m = m0 + rt * 16 + (lane & 15);
-    if (m >= M) continue;
-    long p_raw = 0;
-    if (EPI == GEPI_ROPE) p_raw = ro.pos[m];
+    for (int u = 0; u < U; ++u) v[u] = *(const f16x8*)(lds + G::piece(r0 + G::RS * u, p));
+    if constexpr (EPI == GEPI_STORE) {
+      if (vec && full) {
+        f16x8 rv[U];
+        if (res) {
 #pragma unroll
-    for (int ft = 0; ft < 2; ++ft) {
-      const int nb = n0 + (wv * 2 + ft) * 16 + 4 * (lane >> 4);
-      if (nb >= N) continue;
-      f16x4 yv;
+          for (int u = 0; u < U; ++u)
+            rv[u] = *(const f16x8*)(res + (long)min(m0 + r0 + G::RS * u, M - 1) * ldr + nb);
+        }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) yv[r] = (f16)acc[ft][rt][r];
-      if (EPI == GEPI_STORE) {
-        if (vec && nb + 3 < N) {  // one 8-byte store (and residual load) per lane
-          if (res) yv = yv + *(const f16x4*)(res + (long)m * ldr + nb);
-          *(f16x4*)(y + (long)m * ldy + nb) = yv;
-        } else {
+        for (int u = 0; u < U; ++u) {
+          const int m = m0 + r0 + G::RS * u;
+          if (m < M) *(f16x8*)(y + (long)m * ldy + nb) = res ? v[u] + rv[u] : v[u];
+        }
+      } else {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            if (nb + r < N) {
-              f16 o = yv[r];
-              if (res) o = o + res[(long)m * ldr + nb + r];
-              y[(long)m * ldy + nb + r] = o;
-            }
+        for (int u = 0; u < U; ++u) {
+          const int m = m0 + r0 + G::RS * u;
+          for (int j = 0; m < M && j < 8 && nb + j < N; ++j) {
+            f16 o = v[u][0];
+            if (res) o = o + res[(long)m * ldr + nb + j];
+            y[(long)m * ldy + nb + j] = o;
+            v[u] = __builtin_shufflevector(v[u], v[u], 1, 2, 3, 4, 5, 6, 7, 0);
           }
         }
-      } else if (EPI == GEPI_ROPE) {  // HD % 4 == 0: the 4 features lie in one head
-        const int h = nb / ro.HD, d = nb - h * ro.HD;
-        const bool pval = p_raw >= 0 && p_raw < ro.L;
-        const long p = p_raw < 0 ? 0 : (p_raw >= ro.L ? ro.L - 1 : p_raw);
-        f16x4 o = yv;
-        if (h < ro.Hq + ro.Hk) {
-          const f32x4 cs = *(const f32x4*)(ro.rope + p * ro.HD + d);
-          const float x0 = (float)yv[0], x1 = (float)yv[1], x2 = (float)yv[2], x3 = (float)yv[3];
-          o[0] = (f16)(x0 * cs[0] - x1 * cs[1]);
-          o[1] = (f16)(x1 * cs[0] + x0 * cs[1]);
-          o[2] = (f16)(x2 * cs[2] - x3 * cs[3]);
-          o[3] = (f16)(x3 * cs[2] + x2 * cs[3]);
+      }
+    } else if constexpr (EPI == GEPI_ROPE) {
+      long pr[U];
+      f32x4 cs[U][2];
+#pragma unroll
+      for (int u = 0; u < U; ++u) pr[u] = ro.pos[min(m0 + r0 + G::RS * u, M - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const long pc = pr[u] < 0 ? 0 : (pr[u] >= ro.L ? ro.L - 1 : pr[u]);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) cs[u][q] = *(const f32x4*)(ro.rope + pc * ro.HD + hd[q]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int m = m0 + r0 + G::RS * u;
+        if (m >= M) break;
+        const bool pval = pr[u] >= 0 && pr[u] < ro.L;
+        const int bi = m / ro.S;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          if (nb + 4 * q >= N) break;
+          const int h = hh[q], d = hd[q];
+          f16x4 o = q ? __builtin_shufflevector(v[u], v[u], 4, 5, 6, 7)
+                      : __builtin_shufflevector(v[u], v[u], 0, 1, 2, 3);
+          if (h < ro.Hq + ro.Hk) {
+            const f32x4 c = cs[u][q];
+            const float x0 = (float)o[0], x1 = (float)o[1], x2 = (float)o[2], x3 = (float)o[3];
+            o[0] = (f16)(x0 * c[0] - x1 * c[1]);
+            o[1] = (f16)(x1 * c[0] + x0 * c[1]);
+            o[2] = (f16)(x2 * c[2] - x3 * c[3]);
+            o[3] = (f16)(x3 * c[2] + x2 * c[3]);
+          }
+          if (h < ro.Hq) {
+            *(f16x4*)(ro.q + ((long)m * ro.Hq + h) * ro.HD + d) = o;
+          } else if (pval) {
+            const int kh = h < ro.Hq + ro.Hk ? h - ro.Hq : h - ro.Hq - ro.Hk;
+            f16* dst = h < ro.Hq + ro.Hk ? ro.kc : ro.vc;
+            *(f16x4*)(dst + (((long)bi * ro.Hk + kh) * ro.L + pr[u]) * ro.HD + d) = o;
+          }
         }
-        if (h < ro.Hq) {
-          *(f16x4*)(ro.q + ((long)m * ro.Hq + h) * ro.HD + d) = o;
-        } else if (pval) {
-          const int b = m / ro.S;
-          const int kh = h < ro.Hq + ro.Hk ? h - ro.Hq : h - ro.Hq - ro.Hk;
-          f16* dst = h < ro.Hq + ro.Hk ? ro.kc : ro.vc;
-          *(f16x4*)(dst + (((long)b * ro.Hk + kh) * ro.L + p) * ro.HD + d) = o;
+      }
+    } else {  // pairs (a_j, b_j) with j = nb / 2 ..; N even
+      const bool v8 = full && ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int m = m0 + r0 + G::RS * u;
+        if (m >= M) break;
+        const f16x4 o = silu_mul4(v[u]);
+        f16* dst = y + (long)m * ldy + (nb >> 1);
+        if (v8) {
+          *(f16x4*)dst = o;
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (nb + 2 * q < N) dst[q] = o[q];
         }
-      } else {  // (a_j, b_j, a_j+1, b_j+1) with j = nb / 2; N even
-        const int j = nb >> 1;
-        const float a0 = (float)yv[0], a1 = (float)yv[2];
-        f16x2 o;
-        o.x = (f16)(a0 / (1.0f + expf(-a0))) * yv[1];
-        o.y = (f16)(a1 / (1.0f + expf(-a1))) * yv[3];
-        *(f16x2*)(y + (long)m * ldy + j) = o;
       }
     }
   }
+}
+
+template <int EPI, bool RM, int WN, int WM, int FT, int RT, int NS>
+static int launch_cfg(const f16* x, long ldx, const int8_t* wp, const f16* s, const f16* res,
+                      long ldr, f16* y, long ldy, int M, int N, int K, hipStream_t st,
+                      const RopeOut& ro) {
+  constexpr int BN = 32 * WN * FT, BM = 32 * WM * RT;
+  const int nfb = (N + BN - 1) / BN, nmb = (M + BM - 1) / BM;
+  const long blocks = (long)nfb * nmb;
+  if (blocks > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  hipLaunchKernelGGL((gemm_i8p_kernel<EPI, RM, WN, WM, FT, RT, NS>), dim3((unsigned)blocks),
+                     dim3(64 * WN * WM), 0, st, x, ldx, wp, s, res, ldr, y, ldy, M, N, K, nfb, nmb, ro);
+  return ecd_launch_status();
+}
+
+// The tiles (features x rows, LDS stages).  A launch takes ceil(blocks / 256) rounds, a round about K / 64
+// chunk times plus a fill and an epilogue; in ns, measured over K = 3072 and 8192 with 40 to 2048
+// workgroups; a chunk takes longer when all CUs load at once (`full`: 256 workgroups) than with at
+// most LIGHT of them (`light`).  One feature tile per wave everywhere: with two, the conversion of twice the
+// weights between the same products made every shape 15 to 25% slower.
+struct Tile {
+  int bn, bm, light, full, edge;
+};
+constexpr int LIGHT = 144;
+constexpr Tile TILES[4] = {
+    {256, 128, 580, 920, 2500},  // 1: 8 waves of 32 x 128, 3 stages
+    {128, 128, 385, 570, 1200},  // 2: 4 waves of 32 x 128, 3 stages (two workgroups per CU)
+    {64, 128, 300, 370, 800},    // 3: 4 waves of 32 x 64, 7 stages
+    {64, 64, 255, 280, 600},     // 4: 4 waves of 32 x 32, 12 stages
+};
+
+// The tile of the shortest estimate.  (Of 18 prompt shapes measured with every tile it is the fastest or
+// within 3% of it.)
+static int default_tile(int M, int N, int K) {
+  int best = 1;
+  long tb = 0;
+  for (int i = 0; i < 4; ++i) {
+    const Tile& t = TILES[i];
+    const long blocks = (long)((N + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
+    const long load = blocks <= LIGHT ? 0 : (blocks >= 256 ? 256 - LIGHT : blocks - LIGHT);
+    const long chunk = t.light + (t.full - t.light) * load / (256 - LIGHT);
+    const long est = (blocks + 255) / 256 * ((K >> 6) * chunk + t.edge);
+    if (i == 0 || est < tb) {
+      best = i + 1;
+      tb = est;
+    }
+  }
+  return best;
 }
 
 template <int EPI, bool RM = false>
 static int launch_gemm(const f16* x, long ldx, const int8_t* wp, const f16* s, const f16* res,
                        long ldr, f16* y, long ldy, int M, int N, int K, hipStream_t st,
                        RopeOut ro = RopeOut{}) {
-  const int nfb = (N + GT_N - 1) / GT_N;
-  const int nmb = (M + GT_M - 1) / GT_M;
-  const long blocks = (long)((nfb + 7) / 8) * 8 * nmb;
-  if (blocks > 0x7FFFFFFFL) return ECD_ENOTSUP;
-  hipLaunchKernelGGL((gemm_i8p_kernel<EPI, RM>), dim3((unsigned)blocks), dim3(256), 0, st, x, ldx,
-                     wp, s, res, ldr, y, ldy, M, N, K, nfb, nmb, ro);
-  return ecd_launch_status();
+#define I8_CFG(I, ...)                                                                            \
+  case I:                                                                                         \
+    return launch_cfg<EPI, RM, __VA_ARGS__>(x, ldx, wp, s, res, ldr, y, ldy, M, N, K, st, ro)
+  switch (default_tile(M, N, K)) {
+    I8_CFG(1, 8, 1, 1, 4, 3);
+    I8_CFG(2, 4, 1, 1, 4, 3);
+    I8_CFG(3, 2, 2, 1, 2, 7);
+    I8_CFG(4, 2, 2, 1, 1, 12);
+    default: return ECD_EINVAL;
+  }
+#undef I8_CFG
 }
 
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
