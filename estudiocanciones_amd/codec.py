@@ -696,6 +696,23 @@ class ScalarDecoder:
                 yr = y[b * (ypad + T) + ypad + t0:]
                 self._gemm(cv, c, K, n, n, 0, False, yr, ld, -1)
 
+    def _fusable_unit(self, c1, c2):
+        """True where ecd_codec_unit64 takes a residual unit: 64 channels, 7 causal taps at one
+        dilation that fits the padding, biases and PReLUs."""
+        o = list(c1.off)
+        return (c1.cin == c1.cout == c2.cin == c2.cout == 64 and c1.k == 7 and c2.k == 1 and o[6] == 0
+                and list(c2.off) == [0] and o == [(j - 6) * -o[5] for j in range(7)]
+                and 0 < -o[5] and -6 * o[5] <= min(self.PAD, 64)
+                and None not in (c1.lin.b, c2.lin.b, c1.prelu, c2.prelu))
+
+    def _fusable_tail(self):
+        """True where ecd_codec_post_final takes the PostProcessor and the final conv."""
+        causal = [j - 6 for j in range(7)]
+        return (self.post.cin == self.post.cout == self.final.cin == 64 and self.final.cout == 1
+                and list(self.post.off) == causal and list(self.final.off) == causal
+                and None not in (self.post.lin.b, self.final.lin.b, self.post.prelu)
+                and self.final.prelu is None)
+
     def decode(self, latent: torch.Tensor) -> torch.Tensor:
         """latent [1, T, S * latent_dim] fp16 (one window) -> waveform [S, T * up, num_bands]
         fp16, S = the channel groups (the two stereo channels), up = prod(factors) * 2."""
@@ -717,12 +734,28 @@ class ScalarDecoder:
             # transposed conv: GEMM rows are input steps, each writing s consecutive outputs
             self._gemm(up, a, up.cin, S * T, T, P, True, bb, s * C, P // s)
             T *= s
-            h = self._buf(f"h{i}", S * T, C)
-            for c1, c2 in units:
-                self._gemm(c1, bb, C, S * T, T, P, True, h, C, -1)
-                self._gemm(c2, h, C, S * T, T, 0, False, bb, C, P, res=True)
+            if all(self._fusable_unit(c1, c2) for c1, c2 in units):
+                # one pass per unit, in turn between two padded buffers (a unit's tiles read rows that
+                # their neighbours write)
+                other = self._pbuf(f"u{i}", S, T, C)
+                for c1, c2 in units:
+                    _ffi.call("ecd_codec_unit64", bb.data_ptr(), other.data_ptr(), c1.lin.wp.data_ptr(),
+                              c1.lin.b.data_ptr(), c1.prelu, c2.lin.wp.data_ptr(),
+                              c2.lin.b.data_ptr(), c2.prelu, S, T, P, c1.off[6] - c1.off[5], st)
+                    bb, other = other, bb
+            else:
+                h = self._buf(f"h{i}", S * T, C)
+                for c1, c2 in units:
+                    self._gemm(c1, bb, C, S * T, T, P, True, h, C, -1)
+                    self._gemm(c2, h, C, S * T, T, 0, False, bb, C, P, res=True)
             a = bb
         T2 = 2 * T
+        if self._fusable_tail():
+            y = self._buf("out", S * T2, 1)
+            _ffi.call("ecd_codec_post_final", a.data_ptr(), self.post.lin.wp.data_ptr(),
+                      self.post.lin.b.data_ptr(), self.post.prelu, self.final.lin.wp.data_ptr(),
+                      self.final.lin.b.data_ptr(), y.data_ptr(), S, T, P, st)
+            return y.view(S, T2, 1).clone()
         pb = self._pbuf("post", S, T2, self.post.cout)
         # PostProcessor: 2x row repeat + causal conv, read straight from the padded activation
         self._gemm(self.post, a, self.post.cin, S * T2, T2, P, True, pb, self.post.cout, P, rep=2)

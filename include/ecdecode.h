@@ -442,6 +442,20 @@ int ecd_gemm_f16p_conv(const void* x, long ldx, const void* wp, const float* bia
                        int xpad, int ypad, const int* offsets, int k, int rep, int epi,
                        void* stream);
 
+/* One 64-channel residual unit of the waveform decoder in one pass (sq_codec.py:120-138): y = x +
+ * prelu2(conv1x1(prelu1(conv7(x)))), conv7 causal with dilation dil (taps (j - 6) dil), slopes a1 and a2,
+ * weights packed by ecd_pack_f16 ([64, 448] and [64, 64]), fp32 biases.  x and y are different buffers,
+ * both [S * (pad + T), 64] fp16 with pad zero rows before each sequence (y's pad rows are not
+ * written); 6 dil <= min(pad, 64).  Bit-equal to the two ecd_gemm_f16p_conv calls it replaces. */
+int ecd_codec_unit64(const void* x, void* y, const void* w1, const float* b1, float a1, const void* w2,
+                     const float* b2, float a2, int S, int T, int pad, int dil, void* stream);
+
+/* The waveform decoder's last two stages in one pass (sq_codec.py:140-168, :500-520): nearest 2x repeat,
+ * causal conv7 + PReLU at 64 channels, causal conv7 to one channel.  x [S * (pad + T), 64] fp16
+ * (pad >= 6 zero rows before each sequence), w1 packed [64, 448], wf packed [1, 448], y [S, 2 T] fp16. */
+int ecd_codec_post_final(const void* x, const void* w1, const float* b1, float a1, const void* wf,
+                         const float* bf, void* y, int S, int T, int pad, void* stream);
+
 /* ecd_gemm_f16p_conv with an explicit block tile (cfg as in ecd_gemm_f16p_tuned; 0 = the
  * library's choice).  Replaces nothing in the reference: the launch-shape knob of the waveform
  * decoder's convolutions, for sweeps and for the tests that hold every tile to the same bits. */
