@@ -76,6 +76,13 @@ SIGNATURES = {
                             c_int, _P],
     "ecd_gemm_f16p_conv": [_P, c_long, _P, _P, c_float, _P, c_long, _P, c_long, c_int, c_int,
                            c_int, c_int, c_int, c_int, _P, c_int, c_int, c_int, _P],
+    "ecd_gemm_f16p_splits": [c_int, c_int, c_int],
+    "ecd_gemm_f16p_partial": [_P, c_long, _P, _P, c_int, c_int, c_int, c_int, _P],
+    "ecd_gemm_i8p_splits": [c_int, c_int, c_int],
+    "ecd_gemm_i8p_partial": [_P, c_long, _P, _P, _P, c_int, c_int, c_int, c_int, _P],
+    "ecd_codec_norm_mod_sum": [_P, _P, c_int, _P, _P, c_long, _P, _P, _P, _P, _P, c_long, _P, c_int, c_int,
+                               c_int, c_int, c_float, _P],
+    "ecd_rms_sum": [_P, c_int, _P, _P, _P, _P, c_int, c_int, c_float, _P],
     "ecd_codec_unit64": [_P, _P, _P, _P, c_float, _P, _P, c_float, c_int, c_int, c_int, c_int, _P],
     "ecd_codec_post_final": [_P, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int, _P],
     "ecd_gemm_f16p_conv_tuned": [_P, c_long, _P, _P, c_float, _P, c_long, _P, c_long, c_int, c_int,

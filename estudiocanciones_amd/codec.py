@@ -193,10 +193,14 @@ class LlamaTransformer:
             F2 = max(b.F for b in self.blocks + self.blocks_2)
             cmax = max(self.cin + self.D, D2, self.cin)
             e = lambda *s: torch.empty(*s, device=self.dev, dtype=torch.float16)
+            # fp32 partial sums of the residual branches that _branch splits over K
+            parts = max(M * lin.N * (ks if (ks := _ffi.lib().ecd_gemm_f16p_splits(M, lin.N, lin.K)) > 1 else 0)
+                        for b in self.blocks + self.blocks_2 for lin in (b.o, b.down))
             self._bufs[key] = dict(
                 cols=e(M * 3 * cmax), t1=e(M * D2), x=e(M * D2), y=e(M * D2),
                 q=e(M * D2), k=e(M * D2), v=e(M * D2), o=e(M * D2), h=e(M * D2), m=e(M * F2),
                 out=e(M, self.cout),
+                parts=torch.empty(parts, device=self.dev, dtype=torch.float32),
                 pos=torch.full((M,), T - 1, device=self.dev, dtype=torch.int64))
         return self._bufs[key]
 
@@ -234,10 +238,26 @@ class LlamaTransformer:
         """gate/shift/scale: (table address, vector address); gate None: no residual."""
         R, D = x.shape
         g_tab, g_tm, g_ld = gate if gate is not None else (None, None, 0)
+        if isinstance(h, tuple):  # (partial sums, ways): a product split over K
+            _ffi.call("ecd_codec_norm_mod_sum", x.data_ptr(), h[0].data_ptr(), h[1], g_tab, g_tm, g_ld,
+                      None if w is None else w.data_ptr(), shift[0], shift[1], scale[0], scale[1],
+                      tm_ld, y.data_ptr(), R, T, D, norm, EPS, stream_ptr(self.dev))
+            return
         _ffi.call("ecd_codec_norm_mod", x.data_ptr(), None if h is None else h.data_ptr(),
                   g_tab, g_tm, g_ld, None if w is None else w.data_ptr(), shift[0], shift[1],
                   scale[0], scale[1], tm_ld, y.data_ptr(), R, T, D, norm, EPS,
                   stream_ptr(self.dev))
+
+    def _branch(self, lin, a, buf):
+        """A residual branch's last linear layer (no bias) for the norm that adds it: fp16 rows, or with few
+        rows (fp32 partial sums, ways) of the product split over K."""
+        M, N = a.shape[0], lin.N
+        ks = _ffi.lib().ecd_gemm_f16p_splits(M, N, lin.K)
+        if ks == 1:
+            return lin(a, buf["h"][:M * N].view(M, N))
+        _ffi.call("ecd_gemm_f16p_partial", a.data_ptr(), a.stride(0), lin.wp.data_ptr(),
+                  buf["parts"].data_ptr(), M, N, lin.K, ks, stream_ptr(self.dev))
+        return buf["parts"], ks
 
     def _blocks(self, blocks, x, B, T, tmod, tm_ld, buf):
         """The LlamaTransformerBlock stack; returns the pending gated residual (h, gate) of the
@@ -259,11 +279,11 @@ class LlamaTransformer:
                       self._rope_table(T, HD).data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                       M, T, H, HD, D, st)
             o = prefill_attn(q, k, v, buf["pos"][:M], T, H, H, out=buf["o"][:M * D].view(M, D))
-            ha = bp.o(o, buf["h"][:M * D].view(M, D))
+            ha = self._branch(bp.o, o, buf)
             g_a = ch(2) + (tm_ld,)
             self._norm(x, ha, g_a, bp.mlp_norm, ch(3), ch(4), tm_ld, y, T, 0)
             m = gemm_f16_silu_packed(y, bp.gu, bp.F, D, out=buf["m"][:M * bp.F].view(M, bp.F))
-            h = bp.down(m, buf["h"][:M * D].view(M, D))
+            h = self._branch(bp.down, m, buf)
             gate = ch(5)
         return h, gate
 

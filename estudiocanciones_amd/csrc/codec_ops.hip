@@ -112,9 +112,11 @@ __global__ __launch_bounds__(256) void codec_rope_heads_kernel(
 // g_tm of batch b sits at b * g_ld, sh_tm and sc_tm at b * tm_ld (0: one vector shared by every
 // batch entry).
 // D % 8 == 0, D <= 4096.
-template <int NORM>
+// SUM: the branch arrives as ks fp32 partial sums hp [ks][R, D] (a product split over K), added in order and
+// rounded to the fp16 h.
+template <int NORM, bool SUM>
 __global__ __launch_bounds__(256) void codec_norm_mod_kernel(
-    f16* __restrict__ x, const f16* __restrict__ h, const f16* __restrict__ g_tab,
+    f16* __restrict__ x, const f16* __restrict__ h, const float* __restrict__ hp, int ks, const f16* __restrict__ g_tab,
     const f16* __restrict__ g_tm, long g_ld, const f16* __restrict__ w, const f16* __restrict__ sh_tab,
     const f16* __restrict__ sh_tm, const f16* __restrict__ sc_tab, const f16* __restrict__ sc_tm,
     long tm_ld, f16* __restrict__ y, int T, int D, float eps) {
@@ -129,8 +131,13 @@ __global__ __launch_bounds__(256) void codec_norm_mod_kernel(
     const int c = (threadIdx.x + u * 256) * 8;
     if (c < D) {
       f16x8 xv = *(const f16x8*)(xr + c);
-      if (h) {
-        const f16x8 hv = *(const f16x8*)(h + (long)r * D + c);
+      if (SUM || h) {
+        f16x8 hv;
+        if constexpr (SUM) {
+          hv = sum_partials(hp + (long)r * D + c, (long)gridDim.x * D, ks);
+        } else {
+          hv = *(const f16x8*)(h + (long)r * D + c);
+        }
         const f16x8 gt = *(const f16x8*)(g_tab + c);
         const f16x8 gm = *(const f16x8*)(g_tm + (long)(r / T) * g_ld + c);
 #pragma unroll
@@ -454,28 +461,46 @@ int ecd_codec_rope_heads(const void* qkv, long ldq, const void* tab, void* q, vo
   return ecd_launch_status();
 }
 
+static int norm_mod(void* x, const void* h, const float* hp, int ks, const void* g_tab, const void* g_tm,
+                    long g_ld, const void* w, const void* sh_tab, const void* sh_tm, const void* sc_tab,
+                    const void* sc_tm, long tm_ld, void* y, int R, int T, int D, int norm, float eps,
+                    void* stream) {
+  if (!x || !y || !sh_tab || !sh_tm || !sc_tab || !sc_tm || R <= 0 || T <= 0 || D <= 0 ||
+      (D & 7) || D > 4096 || tm_ld < 0 || (tm_ld & 7) || g_ld < 0 || (g_ld & 7) || (norm != 0 && norm != 1) ||
+      (norm == 0 && !w) || ((h || hp) && (!g_tab || !g_tm)))
+    return ECD_EINVAL;
+  const void* ptrs[] = {x, h, hp, g_tab, g_tm, w, sh_tab, sh_tm, sc_tab, sc_tm, y};
+  for (const void* p : ptrs)
+    if (p && !a16(p)) return ECD_EINVAL;
+#define NM_LAUNCH(NORM, SUM)                                                                              \
+  hipLaunchKernelGGL((codec_norm_mod_kernel<NORM, SUM>), dim3(R), dim3(256), 0, (hipStream_t)stream, (f16*)x, \
+                     (const f16*)h, hp, ks, (const f16*)g_tab, (const f16*)g_tm, g_ld, (const f16*)w,       \
+                     (const f16*)sh_tab, (const f16*)sh_tm, (const f16*)sc_tab, (const f16*)sc_tm, tm_ld,   \
+                     (f16*)y, T, D, eps)
+  if (norm == 0) {
+    if (hp) NM_LAUNCH(0, true); else NM_LAUNCH(0, false);
+  } else {
+    if (hp) NM_LAUNCH(1, true); else NM_LAUNCH(1, false);
+  }
+#undef NM_LAUNCH
+  return ecd_launch_status();
+}
+
+int ecd_codec_norm_mod_sum(void* x, const float* hp, int ks, const void* g_tab, const void* g_tm, long g_ld,
+                           const void* w, const void* sh_tab, const void* sh_tm, const void* sc_tab,
+                           const void* sc_tm, long tm_ld, void* y, int R, int T, int D, int norm, float eps,
+                           void* stream) {
+  if (!hp || ks < 1) return ECD_EINVAL;
+  return norm_mod(x, nullptr, hp, ks, g_tab, g_tm, g_ld, w, sh_tab, sh_tm, sc_tab, sc_tm, tm_ld, y, R, T, D,
+                  norm, eps, stream);
+}
+
 int ecd_codec_norm_mod(void* x, const void* h, const void* g_tab, const void* g_tm, long g_ld,
                        const void* w, const void* sh_tab, const void* sh_tm, const void* sc_tab,
                        const void* sc_tm, long tm_ld, void* y, int R, int T, int D, int norm,
                        float eps, void* stream) {
-  if (!x || !y || !sh_tab || !sh_tm || !sc_tab || !sc_tm || R <= 0 || T <= 0 || D <= 0 ||
-      (D & 7) || D > 4096 || tm_ld < 0 || (tm_ld & 7) || g_ld < 0 || (g_ld & 7) || (norm != 0 && norm != 1) ||
-      (norm == 0 && !w) || (h && (!g_tab || !g_tm)))
-    return ECD_EINVAL;
-  const void* ptrs[] = {x, h, g_tab, g_tm, w, sh_tab, sh_tm, sc_tab, sc_tm, y};
-  for (const void* p : ptrs)
-    if (p && !a16(p)) return ECD_EINVAL;
-  if (norm == 0)
-    hipLaunchKernelGGL(codec_norm_mod_kernel<0>, dim3(R), dim3(256), 0, (hipStream_t)stream,
-                       (f16*)x, (const f16*)h, (const f16*)g_tab, (const f16*)g_tm, g_ld, (const f16*)w,
-                       (const f16*)sh_tab, (const f16*)sh_tm, (const f16*)sc_tab,
-                       (const f16*)sc_tm, tm_ld, (f16*)y, T, D, eps);
-  else
-    hipLaunchKernelGGL(codec_norm_mod_kernel<1>, dim3(R), dim3(256), 0, (hipStream_t)stream,
-                       (f16*)x, (const f16*)h, (const f16*)g_tab, (const f16*)g_tm, g_ld, (const f16*)w,
-                       (const f16*)sh_tab, (const f16*)sh_tm, (const f16*)sc_tab,
-                       (const f16*)sc_tm, tm_ld, (f16*)y, T, D, eps);
-  return ecd_launch_status();
+  return norm_mod(x, h, nullptr, 0, g_tab, g_tm, g_ld, w, sh_tab, sh_tm, sc_tab, sc_tm, tm_ld, y, R, T, D, norm,
+                  eps, stream);
 }
 
 int ecd_codec_cols3(const void* const* seg_ptr, const long* seg_ld, const int* seg_w,

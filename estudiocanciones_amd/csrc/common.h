@@ -150,6 +150,17 @@ __device__ __forceinline__ void rope_pair_f16(float x1, float x2, float co, floa
   o2 = (f16)((float)(f16)(x1 * si) + (float)(f16)(x2 * co));
 }
 
+// fp16 of the sum, in order, of ks fp32 partials at p, p + stride, ..: 8 consecutive values
+__device__ __forceinline__ f16x8 sum_partials(const float* p, long stride, int ks) {
+  f32x4 a = *(const f32x4*)p, b = *(const f32x4*)(p + 4);
+  for (int k = 1; k < ks; ++k) {
+    p += stride;
+    a = a + *(const f32x4*)p;
+    b = b + *(const f32x4*)(p + 4);
+  }
+  return (f16x8){(f16)a[0], (f16)a[1], (f16)a[2], (f16)a[3], (f16)b[0], (f16)b[1], (f16)b[2], (f16)b[3]};
+}
+
 // fp32 -> bf16 bits, round to nearest even (finite inputs).
 __device__ __host__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
   uint32_t u = __builtin_bit_cast(uint32_t, f);

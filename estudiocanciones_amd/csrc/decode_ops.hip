@@ -71,6 +71,45 @@ __global__ __launch_bounds__(256) void rmsnorm_wave_kernel(const f16* __restrict
   }
 }
 
+// A product split over K, its residual and the next RMSNorm: xo = fp16(fp16(sum_k hp[k]) + res) and
+// y = rms(xo) * w (the rounding points of the GEMM's residual epilogue and of rmsnorm_kernel).  One workgroup
+// per row, D % 8 == 0, D <= 4096; res and xo may be the same buffer.
+__global__ __launch_bounds__(256) void rms_sum_kernel(const float* __restrict__ hp, int ks, const f16* res,
+                                                      const f16* __restrict__ w, f16* xo,
+                                                      f16* __restrict__ y, int D, float eps) {
+  __shared__ float part[4];
+  const long r = blockIdx.x;
+  f16x8 v[2];
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = (threadIdx.x + 256 * u) * 8;
+    if (c < D) {
+      v[u] = sum_partials(hp + r * D + c, (long)gridDim.x * D, ks) + *(const f16x8*)(res + r * D + c);
+      *(f16x8*)(xo + r * D + c) = v[u];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float f = (float)v[u][e];
+        ss += f * f;
+      }
+    }
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const float inv = 1.0f / sqrtf((part[0] + part[1] + part[2] + part[3]) / (float)D + eps);
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = (threadIdx.x + 256 * u) * 8;
+    if (c < D) {
+      f16x8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = (f16)((float)v[u][e] * inv);
+      *(f16x8*)(y + r * D + c) = h * *(const f16x8*)(w + c);
+    }
+  }
+}
+
 // ---------------------------------------------------------------- RoPE + KV-cache write
 // One block per row r (batch b = r / S, position p = pos[r]).  Interleaved pairs
 // (x[2i], x[2i+1]) are rotated by the table entry rope[p, i] = (cos, sin); q heads go to
@@ -303,6 +342,16 @@ int ecd_rmsnorm(const void* x, long ldx, const void* w, void* y, long ldy, int R
     default:
       hipLaunchKernelGGL(rmsnorm_kernel<256>, dim3(R), dim3(256), 0, st, xh, ldx, wh, yh, ldy, D, eps);
   }
+  return ecd_launch_status();
+}
+
+int ecd_rms_sum(const float* hp, int ks, const void* res, const void* w, void* xo, void* y, int R, int D,
+                float eps, void* stream) {
+  if (!hp || ks < 1 || !res || !w || !xo || !y || R <= 0 || D <= 0 || (D & 7) || D > 4096 ||
+      (((uintptr_t)hp | (uintptr_t)res | (uintptr_t)w | (uintptr_t)xo | (uintptr_t)y) & 15))
+    return ECD_EINVAL;
+  hipLaunchKernelGGL(rms_sum_kernel, dim3(R), dim3(256), 0, (hipStream_t)stream, hp, ks, (const f16*)res,
+                     (const f16*)w, (f16*)xo, (f16*)y, D, eps);
   return ecd_launch_status();
 }
 

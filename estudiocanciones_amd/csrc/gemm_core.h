@@ -104,6 +104,63 @@ __device__ __forceinline__ f16x4 silu_mul4(const f16x8& v) {
   return o;
 }
 
+// A tile (features x rows) with its measured times in ns: a 64-wide chunk with at most LIGHT workgroups and
+// with 256 (one per CU, all loading), and the fill and epilogue of a round.
+struct Tile {
+  int bn, bm, light, full, edge;
+};
+constexpr int LIGHT = 144;
+
+// Estimate of a launch over nch chunks, K split `ks` ways: rounds of 256 workgroups.
+inline long tile_estimate(const Tile& t, int M, int N, int nch, int ks) {
+  const long blocks = (long)((N + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm) * ks;
+  const long load = blocks <= LIGHT ? 0 : (blocks >= 256 ? 256 - LIGHT : blocks - LIGHT);
+  const long chunk = t.light + (t.full - t.light) * load / (256 - LIGHT);
+  return (blocks + 255) / 256 * ((long)((nch + ks - 1) / ks) * chunk + t.edge);
+}
+
+// The tile of the shortest estimate (0-based), and that estimate.
+inline int best_tile(const Tile* t, int n, int M, int N, int nch, int ks, long* est) {
+  int best = 0;
+  for (int i = 0; i < n; ++i) {
+    const long e = tile_estimate(t[i], M, N, nch, ks);
+    if (i == 0 || e < *est) {
+      best = i;
+      *est = e;
+    }
+  }
+  return best;
+}
+
+// Ways to split K for a product of few rows whose consumer adds fp32 partial sums (1: do not).  A split
+// launch fills CUs that the tiles of one leave idle, at most one workgroup per CU; the ks M N floats that it
+// writes and the consumer reads are taken at 2 floats per ps, its larger edges at 0.5 us.  Product and
+// consuming norm, us, one way -> the rule's ways (best of 1..8):
+//   fp16 weights  187 x 1536 x 1536   11.4 -> 10.1 (2)  10.1 | 187 x 1536 x 4096   17.4 -> 12.3 (3)  12.3
+//                 187 x 3072 x 8192   40.9 -> 28.5 (2)  28.5 | 187 x 3072 x 3072   16.5 -> 16.5 (1)  15.4
+//                  24 x 3072 x 8192   33.8 -> 18.3 (5)  18.1 | 372 x 1536 x 4096   19.1 -> 16.4 (2)  15.4
+//                 372 x 3072 x 8192   55.8 -> 55.8 (1)  45.2 | 744 x 1536 x 4096   25.0 -> 25.0 (1)  25.0
+//   int8 weights   77 x 3072 x 8192   40.7 -> 21.1 (5)  19.6 | 154 x 3072 x 8192   41.1 -> 28.2 (2)  28.2
+//                  77 x 3072 x 3072   19.5 -> 14.1 (5)  13.6 | 154 x 3072 x 3072   20.1 -> 16.6 (2)  16.6
+//                 512 x 3072 x 8192   50.2 -> 50.2 (1)  50.2 | 256 x 3072 x 8192   42.5 -> 30.1 (2)  30.1
+constexpr int SPLIT_MAX = 8;
+inline int split_ways(const Tile* t, int n, const Tile* small, int nsmall, int M, int N, int nch) {
+  long best = 0;
+  best_tile(t, n, M, N, nch, 1, &best);
+  int ks = 1;
+  for (int k = 2; k <= SPLIT_MAX && k * 2 <= nch; ++k)
+    for (int i = 0; i < nsmall; ++i) {
+      const long blocks = (long)((N + small[i].bn - 1) / small[i].bn) * ((M + small[i].bm - 1) / small[i].bm) * k;
+      if (blocks > 256) continue;
+      const long e = tile_estimate(small[i], M, N, nch, k) + (long)k * M * N / 500 + 500;
+      if (e < best) {
+        best = e;
+        ks = k;
+      }
+    }
+  return ks;
+}
+
 template <bool W8, bool RM, int WN, int WM, int FT, int RT, int NS>
 struct GemmTile {
   static constexpr int NW = WN * WM;           // waves
@@ -156,17 +213,21 @@ struct GemmTile {
   // The tile at features n0, rows m0: the fp16 sums (plus bias) of feature n0 + 8 p + j and row m0 + r
   // end at lds[piece(r, p) + j].  sc: the per-feature scales of int8 weights.  RM: w is a row-major
   // [N, K] int8 matrix instead of packed tiles.  Ends with a barrier.
+  // PART: only K chunks c0 .. c0 + cn - 1 (plain rows), whose fp32 sums go to part [M, N] (N % 4 == 0)
+  // instead, straight from the registers.
+  template <bool PART = false>
   static __device__ __forceinline__ void run(f16* lds, const f16* __restrict__ x, long ldx,
                                              const void* __restrict__ wp, const f16* __restrict__ sc,
                                              const float* __restrict__ bias, int M, int N, int K,
-                                             int n0, int m0, const RowMap& rm) {
+                                             int n0, int m0, const RowMap& rm, int c0 = 0, int cn = 0,
+                                             float* __restrict__ part = nullptr) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wv % WN, wm = wv / WN;
-    const int nch = K >> 6;
+    const int nch = PART ? cn : K >> 6;
     const int ntiles = (N + 15) >> 4;
-    const long tile_bytes = RM ? 16L * K : (long)nch * (1024 * WPT);
+    const long tile_bytes = RM ? 16L * K : (long)(K >> 6) * (1024 * WPT);
 
     // DMA sources: weight instruction j of this wave is tile t = i >> 1, half h = i & 1 (int8: tile i) with
     // i = wv + NW j (tiles past N re-read the last tile; their results are never stored); x
@@ -215,6 +276,10 @@ struct GemmTile {
       xb = x + (long)(rm.rep == 2 ? (o >> 1) : o) * ldx;
     };
     if (rm.k) set_tap();
+    if constexpr (PART) {
+      xb += c0 * 64L;
+      wb += (long)c0 * (RM ? 64 : 1024 * WPT);
+    }
     auto next_chunk = [&]() {
       xb += 64;
       wb += RM ? 64 : 1024 * WPT;
@@ -363,6 +428,20 @@ struct GemmTile {
     }
     half(fc, IC<0>{}, lds, fa, IC<0>{}, IC<0>{}, 0);  // (its reads are never used)
 
+    if constexpr (PART) {
+      static_for<0, 4 * FT>([&](auto I) {
+        constexpr int ft = decltype(I)::value >> 2, g = decltype(I)::value & 3;
+        const int n = n0 + (wn * FT + ft) * 32 + 8 * g + 4 * (lane >> 5);
+        static_for<0, RT>([&](auto R) {
+          constexpr int rt = decltype(R)::value;
+          const int m = m0 + (wm * RT + rt) * 32 + (lane & 31);
+          if (m < M && n < N)
+            *(f32x4*)(part + (long)m * N + n) = (f32x4){acc[ft][rt][4 * g], acc[ft][rt][4 * g + 1],
+                                                        acc[ft][rt][4 * g + 2], acc[ft][rt][4 * g + 3]};
+        });
+      });
+      return;
+    }
     // Epilogue.  A lane holds features 8 g + 4 (lane >> 5) .. + 3 (g < 4) of row lane & 31 of each of
     // its tiles.  The rounded sums go through LDS (the stages are free once every wave has read its last
     // fragments), so that a short loop finishes them in 16-byte pieces of consecutive features and

@@ -198,10 +198,6 @@ static int launch_cfg(const f16* x, long ldx, const f16* wp, const float* bias, 
 // ceil(blocks / 256) rounds, a round about K / 64 chunk times plus a fill and an epilogue.  In ns,
 // measured over K = 1536 .. 8192; a chunk takes longer when all CUs load at once (`full`: 256 workgroups)
 // than with at most LIGHT of them (`light`).
-struct Tile {
-  int bn, bm, light, full, edge;
-};
-constexpr int LIGHT = 144;
 constexpr Tile TILES[8] = {
     {256, 256, 1300, 1550, 5000},  // 1: 8 waves of 64 x 128, 2 stages
     {256, 192, 1190, 1450, 3500},  // 2: 8 waves of 64 x 96, 2 stages
@@ -223,20 +219,23 @@ constexpr int MANY_ROWS = 16384;
 // shortest estimate.  (Of 29 shapes measured with every tile it is the fastest or within 10% of it.)
 static int default_cfg(int M, int N, int K) {
   if (M >= MANY_ROWS && N <= 128) return N <= 64 ? 10 : 9;
-  int best = 1;
-  long tb = 0;
-  for (int i = 0; i < 8; ++i) {
-    const Tile& t = TILES[i];
-    const long blocks = (long)((N + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
-    const long load = blocks <= LIGHT ? 0 : (blocks >= 256 ? 256 - LIGHT : blocks - LIGHT);
-    const long chunk = t.light + (t.full - t.light) * load / (256 - LIGHT);
-    const long est = (blocks + 255) / 256 * ((K >> 6) * chunk + t.edge);
-    if (i == 0 || est < tb) {
-      best = i + 1;
-      tb = est;
-    }
-  }
-  return best;
+  long est = 0;
+  return 1 + best_tile(TILES, 8, M, N, K >> 6, 1, &est);
+}
+
+// K split over gridDim.y: fp32 partial sums [gridDim.y][M, N]
+template <int WN, int WM, int FT, int RT, int NS>
+__global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_partial_kernel(
+    const f16* __restrict__ x, long ldx, const f16* __restrict__ wp, float* __restrict__ ws, int M, int N,
+    int K, int nfb, int nmb) {
+  using G = GemmTile<false, false, WN, WM, FT, RT, NS>;
+  __shared__ __align__(16) f16 lds[G::LDS_HALFS];
+  int fb, mb;
+  G::block(nfb, nmb, fb, mb);
+  const RowMap rm = {0, 0, -1, 0, 0, 1, {0, 0, 0, 0, 0, 0, 0, 0}};  // plain rows
+  const int z = blockIdx.y, c0 = (K >> 6) * z / gridDim.y, c1 = (K >> 6) * (z + 1) / gridDim.y;
+  G::template run<true>(lds, x, ldx, wp, nullptr, nullptr, M, N, K, fb * G::BN, mb * G::BM, rm, c0, c1 - c0,
+                        ws + (long)z * M * N);
 }
 
 template <int EPI>
@@ -262,6 +261,16 @@ static int launch_f16(int cfg, const f16* x, long ldx, const f16* wp, const floa
     default: return ECD_EINVAL;
   }
 #undef F16_CFG
+}
+
+template <int WN, int WM, int FT, int RT, int NS>
+static int launch_partial(const f16* x, long ldx, const f16* wp, float* ws, int M, int N, int K, int ks,
+                          hipStream_t st) {
+  const int nfb = (N + 32 * WN * FT - 1) / (32 * WN * FT), nmb = (M + 32 * WM * RT - 1) / (32 * WM * RT);
+  if ((long)nfb * nmb > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  hipLaunchKernelGGL((gemm_f16w_partial_kernel<WN, WM, FT, RT, NS>), dim3((unsigned)(nfb * nmb), ks),
+                     dim3(64 * WN * WM), 0, st, x, ldx, wp, ws, M, N, K, nfb, nmb);
+  return ecd_launch_status();
 }
 
 static int launch_epi(int epi, int cfg, const f16* x, long ldx, const f16* wp, const float* bias,
@@ -383,6 +392,25 @@ int ecd_gemm_f16p_prelu(const void* x, long ldx, const void* wp, const float* bi
                         void* stream) {
   return ecd_gemm_f16p_tuned(x, ldx, wp, bias, slope, res, ldr, y, ldy, M, N, K, F16_PRELU, 0,
                              stream);
+}
+
+int ecd_gemm_f16p_splits(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64)) return 1;
+  return split_ways(TILES, 8, TILES + 6, 2, M, N, K >> 6);
+}
+
+int ecd_gemm_f16p_partial(const void* x, long ldx, const void* wp, float* ws, int M, int N, int K, int ks,
+                          void* stream) {
+  if (!x || !wp || !ws || M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64) || ldx < K || (ldx % 8) ||
+      ks < 1 || ks > SPLIT_MAX || ks > K / 64 || !al16(x) || !al16(wp) || !al16(ws))
+    return ECD_EINVAL;
+  if (!x_offsets_fit(M, ldx)) return ECD_ENOTSUP;
+  long est = 0;
+  const f16 *xh = (const f16*)x, *wh = (const f16*)wp;
+  const hipStream_t st = (hipStream_t)stream;
+  if (best_tile(TILES + 6, 2, M, N, K >> 6, ks, &est) == 0)
+    return launch_partial<2, 2, 1, 2, 5>(xh, ldx, wh, ws, M, N, K, ks, st);
+  return launch_partial<2, 2, 1, 1, 8>(xh, ldx, wh, ws, M, N, K, ks, st);
 }
 
 int ecd_gemm_f16p_silu(const void* x, long ldx, const void* wp, void* mm, long ldm, int M, int F,

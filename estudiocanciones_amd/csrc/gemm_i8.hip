@@ -177,10 +177,6 @@ static int launch_cfg(const f16* x, long ldx, const int8_t* wp, const f16* s, co
 // workgroups; a chunk takes longer when all CUs load at once (`full`: 256 workgroups) than with at
 // most LIGHT of them (`light`).  One feature tile per wave everywhere: with two, the conversion of twice the
 // weights between the same products made every shape 15 to 25% slower.
-struct Tile {
-  int bn, bm, light, full, edge;
-};
-constexpr int LIGHT = 144;
 constexpr Tile TILES[4] = {
     {256, 128, 580, 920, 2500},  // 1: 8 waves of 32 x 128, 3 stages
     {128, 128, 385, 570, 1200},  // 2: 4 waves of 32 x 128, 3 stages (two workgroups per CU)
@@ -191,20 +187,33 @@ constexpr Tile TILES[4] = {
 // The tile of the shortest estimate.  (Of 18 prompt shapes measured with every tile it is the fastest or
 // within 3% of it.)
 static int default_tile(int M, int N, int K) {
-  int best = 1;
-  long tb = 0;
-  for (int i = 0; i < 4; ++i) {
-    const Tile& t = TILES[i];
-    const long blocks = (long)((N + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
-    const long load = blocks <= LIGHT ? 0 : (blocks >= 256 ? 256 - LIGHT : blocks - LIGHT);
-    const long chunk = t.light + (t.full - t.light) * load / (256 - LIGHT);
-    const long est = (blocks + 255) / 256 * ((K >> 6) * chunk + t.edge);
-    if (i == 0 || est < tb) {
-      best = i + 1;
-      tb = est;
-    }
-  }
-  return best;
+  long est = 0;
+  return 1 + best_tile(TILES, 4, M, N, K >> 6, 1, &est);
+}
+
+// K split over gridDim.y: fp32 partial sums [gridDim.y][M, N]
+template <int WN, int WM, int FT, int RT, int NS>
+__global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_partial_kernel(
+    const f16* __restrict__ x, long ldx, const int8_t* __restrict__ wp, const f16* __restrict__ s,
+    float* __restrict__ ws, int M, int N, int K, int nfb, int nmb) {
+  using G = GemmTile<true, false, WN, WM, FT, RT, NS>;
+  __shared__ __align__(16) f16 lds[G::LDS_HALFS];
+  int fb, mb;
+  G::block(nfb, nmb, fb, mb);
+  const RowMap rm = {0, 0, -1, 0, 0, 1, {0, 0, 0, 0, 0, 0, 0, 0}};  // plain rows
+  const int z = blockIdx.y, c0 = (K >> 6) * z / gridDim.y, c1 = (K >> 6) * (z + 1) / gridDim.y;
+  G::template run<true>(lds, x, ldx, wp, s, nullptr, M, N, K, fb * G::BN, mb * G::BM, rm, c0, c1 - c0,
+                        ws + (long)z * M * N);
+}
+
+template <int WN, int WM, int FT, int RT, int NS>
+static int launch_partial(const f16* x, long ldx, const int8_t* wp, const f16* s, float* ws, int M, int N, int K,
+                          int ks, hipStream_t st) {
+  const int nfb = (N + 32 * WN * FT - 1) / (32 * WN * FT), nmb = (M + 32 * WM * RT - 1) / (32 * WM * RT);
+  if ((long)nfb * nmb > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  hipLaunchKernelGGL((gemm_i8p_partial_kernel<WN, WM, FT, RT, NS>), dim3((unsigned)(nfb * nmb), ks),
+                     dim3(64 * WN * WM), 0, st, x, ldx, wp, s, ws, M, N, K, nfb, nmb);
+  return ecd_launch_status();
 }
 
 template <int EPI, bool RM = false>
@@ -278,6 +287,26 @@ int ecd_gemm_i8p_silu(const void* x, long ldx, const void* wp, const void* s, vo
   if (!x_offsets_fit(M, ldx)) return ECD_ENOTSUP;
   return launch_gemm<GEPI_SILU>((const f16*)x, ldx, (const int8_t*)wp, (const f16*)s, nullptr,
                                 0, (f16*)mm, ldm, M, 2 * F, K, (hipStream_t)stream);
+}
+
+int ecd_gemm_i8p_splits(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64)) return 1;
+  return split_ways(TILES, 4, TILES + 2, 2, M, N, K >> 6);
+}
+
+int ecd_gemm_i8p_partial(const void* x, long ldx, const void* wp, const void* s, float* ws, int M, int N, int K,
+                         int ks, void* stream) {
+  if (!x || !wp || !s || !ws || M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64) || ldx < K || (ldx % 8) ||
+      ks < 1 || ks > SPLIT_MAX || ks > K / 64 || !al16(x) || !al16(wp) || !al16(ws))
+    return ECD_EINVAL;
+  if (!x_offsets_fit(M, ldx)) return ECD_ENOTSUP;
+  long est = 0;
+  const f16 *xh = (const f16*)x, *sh = (const f16*)s;
+  const int8_t* wh = (const int8_t*)wp;
+  const hipStream_t st = (hipStream_t)stream;
+  if (best_tile(TILES + 2, 2, M, N, K >> 6, ks, &est) == 0)
+    return launch_partial<2, 2, 1, 2, 7>(xh, ldx, wh, sh, ws, M, N, K, ks, st);
+  return launch_partial<2, 2, 1, 1, 12>(xh, ldx, wh, sh, ws, M, N, K, ks, st);
 }
 
 }  // extern "C"

@@ -37,7 +37,7 @@ import torch
 
 from . import _ffi
 from .kernels import (_attn, _attn_combine, _rope_cache, _silu_mul, cdiv, embed_gemv_packed,
-                      gemm_packed, gemm_silu_packed, gemv_packed_splitk, prefill_attn,
+                      gemm_packed, gemm_rms_packed, gemm_silu_packed, gemv_packed_splitk, prefill_attn,
                       gemm_rope_packed, gemv_packed, int8_mm, layer_head, layer_stack,
                       layer_stack_plan, layer_stack_supported, layer_tail, layer_tail_supported,
                       layer_tail_ws_bytes, next_power_of_2,
@@ -395,15 +395,17 @@ class Stack:
         reference's dense numerics (M > 16); RMSNorm, RoPE + cache write and the causal
         attention (row r attends [0, pos[r]]) use the decode kernels."""
         R = x.shape[0]
-        for b in self.blocks:
+        norms = [b.n1 for b in self.blocks[1:]] + [self.norm]
+        y = krms(x, self.blocks[0].n1 if self.blocks else self.norm)
+        for b, next_norm in zip(self.blocks, norms):
             Hq, Hk, HD, L = b.h, b.kvh, b.hd, b.kc.shape[2]
             q = torch.empty(R, Hq * HD, device=x.device, dtype=x.dtype)
             if HD % 4 == 0:
                 # q | k | v GEMM with RoPE and the cache write in its epilogue
-                gemm_rope_packed(krms(x, b.n1), b.qkv.qp, b.qkv.sp, self.rope, pos, q, b.kc,
+                gemm_rope_packed(y, b.qkv.qp, b.qkv.sp, self.rope, pos, q, b.kc,
                                  b.vc, S, Hq, Hk, L, HD, b.qkv.K)
             else:
-                qkv = gemm_packed(krms(x, b.n1), b.qkv.qp, b.qkv.sp, b.qkv.N, b.qkv.K)
+                qkv = gemm_packed(y, b.qkv.qp, b.qkv.sp, b.qkv.N, b.qkv.K)
                 _rope_cache[(R, Hq + Hk)](qkv, self.rope, pos, q, b.kc, b.vc, S, Hq, Hk, L,
                                           HD=HD, HALF=next_power_of_2(HD // 2))
             if HD == 128 and Hq // Hk <= 4:
@@ -413,10 +415,10 @@ class Stack:
                 # one split per row: a prompt row attends at most the prompt (no empty splits,
                 # no combine pass); the rows themselves give the parallelism
                 o = self._attention(b, q, pos, S, splits=1)
-            x = gemm_packed(o, b.o.qp, b.o.sp, b.o.N, b.o.K, res=x)
-            mm = gemm_silu_packed(krms(x, b.n2), b.w13.qp, b.w13.sp, b.w13.N // 2, b.w13.K)
-            x = gemm_packed(mm, b.w2.qp, b.w2.sp, b.w2.N, b.w2.K, res=x)
-        return krms(x, self.norm)
+            x, y = gemm_rms_packed(o, b.o.qp, b.o.sp, b.o.N, b.o.K, x, b.n2)
+            mm = gemm_silu_packed(y, b.w13.qp, b.w13.sp, b.w13.N // 2, b.w13.K)
+            x, y = gemm_rms_packed(mm, b.w2.qp, b.w2.sp, b.w2.N, b.w2.K, x, next_norm)
+        return y
 
     def decode(self, x, pos, S, final_norm=True, o0=None):
         """Fast path for few rows (app/engine.py:180-211): x [R, D] with R = B*S (row r -> batch

@@ -410,6 +410,32 @@ def gemm_packed(x, wp, s, N, K, res=None):
     return y
 
 
+def gemm_rms_packed(x, wp, s, N, K, res, nw, eps=1e-5):
+    """(h, rms(h, nw)) with h = gemm_packed(x, wp, s, N, K, res): a residual branch and the next layer's
+    norm.  With few rows the product is split over K and one kernel adds the fp32 partial sums and the
+    residual and forms the norm; the rounding points are the same."""
+    M = x.shape[0]
+    ks = _ffi.lib().ecd_gemm_i8p_splits(M, N, K) if N <= 4096 and res.is_contiguous() and \
+        res.data_ptr() % 16 == 0 and nw.data_ptr() % 16 == 0 else 1
+    if ks == 1:
+        h = gemm_packed(x, wp, s, N, K, res)
+        return h, rms(h, nw, eps)
+    _check_x(x, K, "gemm_rms_packed")
+    _f16(res, "gemm_rms_packed res")
+    _f16(nw, "gemm_rms_packed nw")
+    if res.shape != (M, N) or nw.numel() != N or not nw.is_contiguous():
+        raise ValueError("gemm_rms_packed: res must be [M, N] and nw [N]")
+    ws = torch.empty(ks * M * N, device=x.device, dtype=torch.float32)
+    h = torch.empty(M, N, device=x.device, dtype=torch.float16)
+    y = torch.empty_like(h)
+    st = stream_ptr(x.device)
+    _ffi.call("ecd_gemm_i8p_partial", x.data_ptr(), x.stride(0), wp.data_ptr(), s.data_ptr(), ws.data_ptr(), M, N,
+              K, ks, st)
+    _ffi.call("ecd_rms_sum", ws.data_ptr(), ks, res.data_ptr(), nw.data_ptr(), h.data_ptr(), y.data_ptr(), M, N,
+              float(eps), st)
+    return h, y
+
+
 def gemm_silu_packed(x, wp, s, F, K):
     """_silu_mul(int8_mm(x, w1|w3, s)) for many rows on row-interleaved packed w1|w3
     (pack_i8(..., interleave=True)) -> [M, F]."""

@@ -442,6 +442,24 @@ int ecd_gemm_f16p_conv(const void* x, long ldx, const void* wp, const float* bia
                        int xpad, int ypad, const int* offsets, int k, int rep, int epi,
                        void* stream);
 
+/* A product of few rows split over K, for consumers that add the fp32 partial sums: ecd_gemm_*_splits gives
+ * the number of ways (1: use the ordinary call), ecd_gemm_*_partial writes ws [ks][M, N] (N % 64 == 0,
+ * ks <= 8, 16-byte aligned; no bias, scale or residual).  ecd_codec_norm_mod_sum is ecd_codec_norm_mod with
+ * h = fp16(sum of hp [ks][R, D] in order); ecd_rms_sum adds res, writes the sum to xo and its RMSNorm to y
+ * (the reference's residual add and next norm, app/engine.py:141-153; D % 8 == 0, D <= 4096). */
+int ecd_gemm_f16p_splits(int M, int N, int K);
+int ecd_gemm_f16p_partial(const void* x, long ldx, const void* wp, float* ws, int M, int N, int K, int ks,
+                          void* stream);
+int ecd_gemm_i8p_splits(int M, int N, int K);
+int ecd_gemm_i8p_partial(const void* x, long ldx, const void* wp, const void* s, float* ws, int M, int N, int K,
+                         int ks, void* stream);
+int ecd_codec_norm_mod_sum(void* x, const float* hp, int ks, const void* g_tab, const void* g_tm, long g_ld,
+                           const void* w, const void* sh_tab, const void* sh_tm, const void* sc_tab,
+                           const void* sc_tm, long tm_ld, void* y, int R, int T, int D, int norm, float eps,
+                           void* stream);
+int ecd_rms_sum(const float* hp, int ks, const void* res, const void* w, void* xo, void* y, int R, int D,
+                float eps, void* stream);
+
 /* One 64-channel residual unit of the waveform decoder in one pass (sq_codec.py:120-138): y = x +
  * prelu2(conv1x1(prelu1(conv7(x)))), conv7 causal with dilation dil (taps (j - 6) dil), slopes a1 and a2,
  * weights packed by ecd_pack_f16 ([64, 448] and [64, 64]), fp32 biases.  x and y are different buffers,
