@@ -16,6 +16,7 @@
 //                    registers); lane l ends with the scores of its row for slots
 //                    t0 + 16 j + 4 (l >> 4) + i, i < 4;
 //   softmax          per row on its 16 lanes' values, reductions across the 4 lane groups;
+//                    the running sum kept per lane until the end;
 //                    the mask only on tiles that reach past a row's position, the rescale of
 //                    the running state only when a row's maximum grew;
 //   O^T += V^T . P^T v_mfma_f32_16x16x32_f16 with P^T as B straight from the softmax registers:
@@ -34,13 +35,36 @@ namespace ecd {
 constexpr int PA_QB = 64;            // rows per workgroup (4 waves x 16)
 constexpr int PA_KT = 64;            // cache slots per tile
 
+// maximum / sum over the four 16-lane groups that share a row: lane swaps in the VALU, no LDS round trip
+__device__ __forceinline__ float row_max(float v) {
+  auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float row_sum(float v) {
+  auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 // V^T word (d, slot pair w) lives at d * 32 + (w ^ vt_swz(d)): the swizzle keeps word pairs
 // together (8-byte fragment reads), puts the fragment reads of a half-wave (16 d rows x 2 lane
 // groups) on distinct banks and keeps the staging writes at most 2-way conflicted
 __device__ __forceinline__ int vt_swz(int d) { return 4 * (((d >> 1) ^ (d >> 3)) & 7); }
 
+// Bound by vector instructions (16 scores per lane and tile: exponentials, their arguments, sums, fp16
+// pairs), then by the chain of one tile; two tiles of loads in flight, two LDS buffers and 128-slot tiles
+// each measured no faster or slower.  The minimum of waves per SIMD in the launch bounds keeps O^T in
+// vector registers: with 512 registers to give, the compiler puts it into accumulation registers and moves
+// it to and fro in each tile.  It stops where a minimum would spill (G HD > 256).  us with 24 heads, before
+// this, the lane swaps, the row sums kept per lane and the 32-bit load offsets -> with them:
+//   2 x 744 rows, head_dim 64   25.9 -> 22.7     head_dim 128   51.3 -> 43.8
+//   1 x 1500 rows, head_dim 64  43.4 -> 36.6     1 x 187 rows    6.2 ->  5.5
+//   causal, 24 heads on 8, head_dim 128: 8 x 256 rows 21.3 -> 19.7, 2 x 77 rows 10.2 -> 9.6
 template <int HD, int G>
-__global__ __launch_bounds__(256) void prefill_attn_kernel(
+__global__ __launch_bounds__(256, G * HD <= 64 ? 4 : G * HD <= 256 ? 2 : 1) void prefill_attn_kernel(
     const f16* __restrict__ q, const f16* __restrict__ kc, const f16* __restrict__ vc,
     const int64_t* __restrict__ pos, f16* __restrict__ o, int S, int Hq, int Hk, int L,
     float scale) {
@@ -103,17 +127,19 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
   // slot (finite values, masked below).
   f16x8 kr[NK], vr[NV][2];
   auto load_tile = [&](int t0) {
+    const f16 *kt = kb + (long)t0 * HD, *vs = vb + (long)t0 * HD;
+    const int last = L - 1 - t0;  // >= 0: a tile starts below the last attended slot
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
       const int c = tid + 256 * i;
-      kr[i] = *(const f16x8*)(kb + (long)min(t0 + c / DCH, L - 1) * HD + 8 * (c % DCH));
+      kr[i] = *(const f16x8*)(kt + (unsigned)(min(c / DCH, last) * HD + 8 * (c % DCH)));
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int u = tid + 256 * i;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        vr[i][h] = *(const f16x8*)(vb + (long)min(t0 + 2 * (u / DCH) + h, L - 1) * HD + 8 * (u % DCH));
+        vr[i][h] = *(const f16x8*)(vs + (unsigned)(min(2 * (u / DCH) + h, last) * HD + 8 * (u % DCH)));
     }
   };
   // K rows as they are; V transposed into words {V[2w][d], V[2w + 1][d]}
@@ -179,9 +205,7 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sacc[g][j][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run[g], mx);
+      const float m_new = fmaxf(m_run[g], row_max(mx));
       const float mb = m_new == -INFINITY ? 0.f : m_new * c2;  // no slot attended yet: p = 0
       float ps = 0.f;
 #pragma unroll
@@ -192,8 +216,6 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
           ps += pr;
           pb[g][j >> 1][4 * (j & 1) + i] = (f16)pr;
         }
-      ps += __shfl_xor(ps, 16, 64);
-      ps += __shfl_xor(ps, 32, 64);
       if (__any(m_new != m_run[g])) {  // alpha = 1 exactly where the maximum did not move
         asm volatile("" ::: "memory");  // keep this a branch: most tiles skip it
         const float alpha = __builtin_amdgcn_exp2f(m_run[g] * c2 - mb);
@@ -232,10 +254,11 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
   }
 
   // O = O^T / l: lane holds row s, d = 16 dt + 4 grp + i
-  if (!rowok) return;
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    const float inv = l_run[g] > 0.f ? 1.f / l_run[g] : 0.f;
+    const float l = row_sum(l_run[g]);  // each lane's share so far; all rows of the wave take part
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    if (!rowok) continue;
     f16* dst = o + r * (long)Hq * HD + (long)(kh * G + g) * HD + 4 * grp;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
