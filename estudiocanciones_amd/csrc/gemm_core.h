@@ -119,12 +119,17 @@ inline long tile_estimate(const Tile& t, int M, int N, int nch, int ks) {
   return (blocks + 255) / 256 * ((long)((nch + ks - 1) / ks) * chunk + t.edge);
 }
 
-// The tile of the shortest estimate (0-based), and that estimate.
+// The loads' weight offsets are 32-bit from a workgroup's first feature: its bn features of K 16-bit values
+// (int8 weights: half of that) must stay below 4 GiB.
+inline bool w_offsets_fit(int bn, int nch) { return (long)bn * nch * 128 <= 0xFFFFFFFFL; }
+
+// The tile of the shortest estimate (0-based) among those whose weight offsets fit, and that estimate.
 inline int best_tile(const Tile* t, int n, int M, int N, int nch, int ks, long* est) {
-  int best = 0;
+  int best = n - 1;  // the narrowest: the launch refuses it if even that does not fit
+  *est = 0x7FFFFFFFFFFFFFFFL;
   for (int i = 0; i < n; ++i) {
     const long e = tile_estimate(t[i], M, N, nch, ks);
-    if (i == 0 || e < *est) {
+    if (w_offsets_fit(t[i].bn, nch) && e < *est) {
       best = i;
       *est = e;
     }

@@ -187,7 +187,7 @@ static int launch_cfg(const f16* x, long ldx, const f16* wp, const float* bias, 
   const int nfb = (N + BN - 1) / BN;
   const int nmb = (M + BM - 1) / BM;
   const long blocks = (long)nfb * nmb;
-  if (blocks > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  if (blocks > 0x7FFFFFFFL || !w_offsets_fit(32 * WN * FT, K >> 6)) return ECD_ENOTSUP;
   hipLaunchKernelGGL((gemm_f16w_kernel<EPI, WN, WM, FT, RT, NS>), dim3((unsigned)blocks),
                      dim3(64 * WN * WM), 0, st, x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K,
                      nfb, nmb, rm, ro);
@@ -267,7 +267,7 @@ template <int WN, int WM, int FT, int RT, int NS>
 static int launch_partial(const f16* x, long ldx, const f16* wp, float* ws, int M, int N, int K, int ks,
                           hipStream_t st) {
   const int nfb = (N + 32 * WN * FT - 1) / (32 * WN * FT), nmb = (M + 32 * WM * RT - 1) / (32 * WM * RT);
-  if ((long)nfb * nmb > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  if ((long)nfb * nmb > 0x7FFFFFFFL || !w_offsets_fit(32 * WN * FT, K >> 6)) return ECD_ENOTSUP;
   hipLaunchKernelGGL((gemm_f16w_partial_kernel<WN, WM, FT, RT, NS>), dim3((unsigned)(nfb * nmb), ks),
                      dim3(64 * WN * WM), 0, st, x, ldx, wp, ws, M, N, K, nfb, nmb);
   return ecd_launch_status();

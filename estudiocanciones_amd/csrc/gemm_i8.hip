@@ -166,7 +166,7 @@ static int launch_cfg(const f16* x, long ldx, const int8_t* wp, const f16* s, co
   constexpr int BN = 32 * WN * FT, BM = 32 * WM * RT;
   const int nfb = (N + BN - 1) / BN, nmb = (M + BM - 1) / BM;
   const long blocks = (long)nfb * nmb;
-  if (blocks > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  if (blocks > 0x7FFFFFFFL || !w_offsets_fit(32 * WN * FT, K >> 6)) return ECD_ENOTSUP;
   hipLaunchKernelGGL((gemm_i8p_kernel<EPI, RM, WN, WM, FT, RT, NS>), dim3((unsigned)blocks),
                      dim3(64 * WN * WM), 0, st, x, ldx, wp, s, res, ldr, y, ldy, M, N, K, nfb, nmb, ro);
   return ecd_launch_status();
@@ -210,7 +210,7 @@ template <int WN, int WM, int FT, int RT, int NS>
 static int launch_partial(const f16* x, long ldx, const int8_t* wp, const f16* s, float* ws, int M, int N, int K,
                           int ks, hipStream_t st) {
   const int nfb = (N + 32 * WN * FT - 1) / (32 * WN * FT), nmb = (M + 32 * WM * RT - 1) / (32 * WM * RT);
-  if ((long)nfb * nmb > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  if ((long)nfb * nmb > 0x7FFFFFFFL || !w_offsets_fit(32 * WN * FT, K >> 6)) return ECD_ENOTSUP;
   hipLaunchKernelGGL((gemm_i8p_partial_kernel<WN, WM, FT, RT, NS>), dim3((unsigned)(nfb * nmb), ks),
                      dim3(64 * WN * WM), 0, st, x, ldx, wp, s, ws, M, N, K, nfb, nmb);
   return ecd_launch_status();
@@ -244,7 +244,7 @@ static bool x_offsets_fit(int M, long ldx) { return (long)M * ldx * 2 < 0x7FFFFF
 int gemm_i8_rowmajor(const f16* x, long ldx, const int8_t* w, const f16* s, const f16* res,
                      long ldr, f16* y, long ldy, int M, int N, int K, hipStream_t st) {
   if ((K % 64) || (ldx % 8) || !al16(x) || !al16(w) || !x_offsets_fit(M, ldx) ||
-      16L * K >= 0x7FFFFFFFL)
+      !w_offsets_fit(64, K >> 6))
     return 1;
   return launch_gemm<GEPI_STORE, true>(x, ldx, w, s, res, ldr, y, ldy, M, N, K, st);
 }

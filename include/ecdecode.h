@@ -379,7 +379,7 @@ int ecd_layer_stack(const void* plan, int nl, const void* o, const void* xin, co
  * prompt pass (app/engine.py:123-153, 174-178).  MFMA-tiled 128 x 128 per workgroup.
  *   x [M, K] fp16 (row stride ldx, 16-byte aligned, K % 64 == 0); wp = ecd_pack_i8(w);
  *   s [N] fp16; res [M, N] (row stride ldr) or NULL; y [M, N] (row stride ldy).
- *   ECD_ENOTSUP when M * ldx * 2 bytes reach 2 GiB (32-bit per-lane load offsets). */
+ *   ECD_ENOTSUP when M * ldx * 2 bytes reach 2 GiB or K exceeds 2^25 (32-bit per-lane load offsets). */
 int ecd_gemm_i8p(const void* x, long ldx, const void* wp, const void* s, const void* res,
                  long ldr, void* y, long ldy, int M, int N, int K, void* stream);
 
@@ -410,7 +410,7 @@ int ecd_gemm_i8p_rope(const void* x, long ldx, const void* wp, const void* s, co
  *   ecd_gemm_f16p_silu: w packed with interleave (gate | up), mm[m, j] =
  *                       fp16(fp16(silu(g)) * u) with g, u the fp16 GEMM outputs (LlamaMLP,
  *                       transformer.py:181-184).
- * x [M, K] fp16 (row stride ldx, 16-byte aligned, K % 64 == 0); ECD_ENOTSUP when M * ldx * 2
+ * x [M, K] fp16 (row stride ldx, 16-byte aligned, K % 64 == 0); ECD_ENOTSUP when K exceeds 2^25 or M * ldx * 2
  * bytes reach 2 GiB. */
 long ecd_packed_bytes_f16(int N, int K);
 int ecd_pack_f16(const void* w, int N, int K, int interleave, void* out, void* stream);
