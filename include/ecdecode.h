@@ -376,7 +376,7 @@ int ecd_layer_stack(const void* plan, int nl, const void* o, const void* xin, co
 
 /* Prompt-pass GEMM (many rows) on packed weights: y = fp16(x @ fp16(q * s)^T) (+ res as an
  * fp16 add) -- the dense numerics of int8_mm for M > 16 (app/kernels.py:46-49), used by the
- * prompt pass (app/engine.py:123-153, 174-178).  MFMA-tiled 128 x 128 per workgroup.
+ * prompt pass (app/engine.py:123-153, 174-178).  MFMA-tiled, the tile by shape.
  *   x [M, K] fp16 (row stride ldx, 16-byte aligned, K % 64 == 0); wp = ecd_pack_i8(w);
  *   s [N] fp16; res [M, N] (row stride ldr) or NULL; y [M, N] (row stride ldy).
  *   ECD_ENOTSUP when M * ldx * 2 bytes reach 2 GiB or K exceeds 2^25 (32-bit per-lane load offsets). */
