@@ -117,10 +117,13 @@ __device__ __forceinline__ void wait_vm0() { wait_vm<0>(); }
 // per-lane byte offset below 2^31) into LDS at dst + 16 * lane (dst uniform).  Issued from
 // inline asm with M0 (the instruction's LDS base) saved and restored around it: with the
 // compiler's builtin every later LDS read would wait for all outstanding DMA (vmcnt 0).
+// A vector instruction that writes a scalar register (readfirstlane, or the reload of a spilled one) needs
+// five wait states before a memory instruction that reads it, and the compiler does not see the load in
+// here: the two M0 moves and s_nop 2 are those five, whatever comes before.
 __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, void* dst) {
   const uint32_t la = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)dst;
   uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 2\n\t"
                "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(off), "s"(base), "s"(la) : "memory");
 }
@@ -128,12 +131,14 @@ __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, void* 
 // The same with the LDS address given as a uniform byte address plus a constant, and M0 left
 // changed: three instructions instead of six where a loop issues many.  The compiler keeps nothing
 // in M0 (it is not allocatable, and no other instruction of these kernels reads it).
+// Where the compiler holds the uniform base in vector registers its readfirstlane may stand right before:
+// the M0 write and s_nop 3 are the five wait states.
 template <int IMM>
 __device__ __forceinline__ void lds_dma16_at(const void* base, uint32_t off, uint32_t lds) {
   const uint64_t b = (uint64_t)base;  // uniform; said again, since it may come through a vector register
   const uint64_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) |
                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32;
-  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1"
                : : "v"(off), "s"(u), "s"(lds), "i"(IMM) : "memory", "scc");
 }
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {

@@ -625,11 +625,11 @@ constexpr int stage_end() {
   return n0 >= CW ? s0 + 8192 * CW : e0 + CW * 1024 + 8192 * (CW - n0);
 }
 
-// One LDS DMA of 16 bytes per lane, nontemporal (lds_dma16 with the nt bit).
+// One LDS DMA of 16 bytes per lane, nontemporal (lds_dma16 with the nt bit, the same wait states).
 __device__ __forceinline__ void lds_dma16_nt(const void* base, uint32_t off, void* dst) {
   const uint32_t la = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)dst;
   uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 2\n\t"
                "global_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(off), "s"(base), "s"(la) : "memory");
 }
