@@ -45,9 +45,6 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
   G::block(nfb, nmb, fb, mb);
   const int n0 = fb * G::BN, m0 = mb * G::BM;
   G::run(lds, x, ldx, wp, nullptr, bias, M, N, K, n0, m0, rm);
-  // 16-byte rows of y (and res) take one store per piece
-  const bool vec = ((ldy & 7) == 0) && (((uintptr_t)y & 15) == 0) &&
-                   (!res || (((ldr & 7) == 0) && (((uintptr_t)res & 15) == 0)));
   constexpr int U = G::U;
   const int p = threadIdx.x % G::PR, nb = n0 + 8 * p;
   if (nb >= N) return;
@@ -78,9 +75,9 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
         m[u] = rm.ypad >= 0 ? seq_row(mm, rm.T, rm.ypad) : mm;
       }
       f16x8 rv[U];
-      if (res && vec && full) {
+      if (res && full) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) rv[u] = *(const f16x8*)(res + m[u] * ldr + nb);
+        for (int u = 0; u < U; ++u) rv[u] = *(const f16x8u*)(res + m[u] * ldr + nb);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -93,16 +90,10 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[u][j] = (f16)((float)v[u][j] * alpha);
         }
-        if (vec && full) {
-          *(f16x8*)(y + m[u] * ldy + nb) = res ? v[u] + rv[u] : v[u];
-        } else {
-          for (int j = 0; j < 8 && nb + j < N; ++j) {
-            f16 o = v[u][0];
-            if (res) o = o + res[m[u] * ldr + nb + j];
-            y[m[u] * ldy + nb + j] = o;
-            v[u] = __builtin_shufflevector(v[u], v[u], 1, 2, 3, 4, 5, 6, 7, 0);
-          }
-        }
+        if (full)
+          *(f16x8u*)(y + m[u] * ldy + nb) = res ? v[u] + rv[u] : v[u];
+        else
+          store_tail(y + m[u] * ldy + nb, res ? res + m[u] * ldr + nb : nullptr, v[u], N - nb);
       }
     } else if constexpr (EPI == F16_ROPE) {
       int rb[U], t[U];
@@ -138,15 +129,14 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
         }
       }
     } else {  // pairs (a_j, b_j) with j = nb / 2 ..; N even
-      const bool v8 = full && ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int mm = m0 + r0 + G::RS * u;
         if (mm >= M) break;
         const f16x4 o = silu_mul4(v[u]);
         f16* dst = y + (long)mm * ldy + (nb >> 1);
-        if (v8) {
-          *(f16x4*)dst = o;
+        if (full) {
+          *(f16x4u*)dst = o;
         } else {
 #pragma unroll
           for (int q = 0; q < 4; ++q)

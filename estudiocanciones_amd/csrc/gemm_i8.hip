@@ -53,8 +53,6 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_kernel(
   const int n0 = fb * G::BN, m0 = mb * G::BM;
   const RowMap rm = {0, 0, -1, 0, 0, 1, {0, 0, 0, 0, 0, 0, 0, 0}};  // plain rows
   G::run(lds, x, ldx, wp, s, nullptr, M, N, K, n0, m0, rm);
-  const bool vec = ((ldy & 7) == 0) && (((uintptr_t)y & 15) == 0) &&
-                   (!res || (((ldr & 7) == 0) && (((uintptr_t)res & 15) == 0)));
   constexpr int U = G::U;
   const int p = threadIdx.x % G::PR, nb = n0 + 8 * p;
   if (nb >= N) return;
@@ -75,29 +73,20 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_kernel(
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = *(const f16x8*)(lds + G::piece(r0 + G::RS * u, p));
     if constexpr (EPI == GEPI_STORE) {
-      if (vec && full) {
-        f16x8 rv[U];
-        if (res) {
+      f16x8 rv[U];
+      if (res && full) {
 #pragma unroll
-          for (int u = 0; u < U; ++u)
-            rv[u] = *(const f16x8*)(res + (long)min(m0 + r0 + G::RS * u, M - 1) * ldr + nb);
-        }
+        for (int u = 0; u < U; ++u)
+          rv[u] = *(const f16x8u*)(res + (long)min(m0 + r0 + G::RS * u, M - 1) * ldr + nb);
+      }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int m = m0 + r0 + G::RS * u;
-          if (m < M) *(f16x8*)(y + (long)m * ldy + nb) = res ? v[u] + rv[u] : v[u];
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int m = m0 + r0 + G::RS * u;
-          for (int j = 0; m < M && j < 8 && nb + j < N; ++j) {
-            f16 o = v[u][0];
-            if (res) o = o + res[(long)m * ldr + nb + j];
-            y[(long)m * ldy + nb + j] = o;
-            v[u] = __builtin_shufflevector(v[u], v[u], 1, 2, 3, 4, 5, 6, 7, 0);
-          }
-        }
+      for (int u = 0; u < U; ++u) {
+        const int m = m0 + r0 + G::RS * u;
+        if (m >= M) break;
+        if (full)
+          *(f16x8u*)(y + (long)m * ldy + nb) = res ? v[u] + rv[u] : v[u];
+        else
+          store_tail(y + (long)m * ldy + nb, res ? res + (long)m * ldr + nb : nullptr, v[u], N - nb);
       }
     } else if constexpr (EPI == GEPI_ROPE) {
       long pr[U];
@@ -140,15 +129,14 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_kernel(
         }
       }
     } else {  // pairs (a_j, b_j) with j = nb / 2 ..; N even
-      const bool v8 = full && ((ldy & 3) == 0) && (((uintptr_t)y & 7) == 0);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int m = m0 + r0 + G::RS * u;
         if (m >= M) break;
         const f16x4 o = silu_mul4(v[u]);
         f16* dst = y + (long)m * ldy + (nb >> 1);
-        if (v8) {
-          *(f16x4*)dst = o;
+        if (full) {
+          *(f16x4u*)dst = o;
         } else {
 #pragma unroll
           for (int q = 0; q < 4; ++q)
