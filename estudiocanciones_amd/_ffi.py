@@ -65,6 +65,8 @@ SIGNATURES = {
     "ecd_gemv_i8p_splitk": [_P, c_long, _P, _P, _P, c_long, _P, c_long, c_int, c_int, c_int, c_int,
                             _P, c_int, _P],
     "ecd_gemm_i8p": [_P, c_long, _P, _P, _P, c_long, _P, c_long, c_int, c_int, c_int, _P],
+    "ecd_gemm_i8p_tile": [c_int, c_int, c_int],
+    "ecd_gemm_i8p_tuned": [_P, c_long, _P, _P, _P, c_long, _P, c_long, c_int, c_int, c_int, c_int, c_int, _P],
     "ecd_gemm_i8p_silu": [_P, c_long, _P, _P, _P, c_long, c_int, c_int, c_int, _P],
     "ecd_gemm_i8p_rope": [_P, c_long, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int,
                           c_int, c_int, c_int, _P],

@@ -19,8 +19,8 @@
 // (M = 154; N, K): (5120, 3072) 36.5 -> 17.1, (3072, 3072) 30.4 -> 16.4, (16384, 3072) 39.4 -> 27.7,
 // (3072, 8192) 91.6 -> 35.7.  At 2048 rows it is bound
 // by the products, the conversion and the LDS reads together: (3072, 3072) 46.6 -> 42.5,
-// (16384, 3072) 197 -> 192, (3072, 8192) 110 -> 102 (1.01 PFLOP/s); at 4096 rows (16384, 3072) 442 -> 397,
-// but (5120, 3072) 131 -> 138 and (3072, 8192) 202 -> 214, where 256 x 128 tiles make 1.5 rounds.
+// (16384, 3072) 197 -> 192, (3072, 8192) 110 -> 102 (1.01 PFLOP/s); at 4096 rows (3072, 3072) 81.9 -> 77.8,
+// (5120, 3072) 132.9 -> 130.4, (16384, 3072) 487 -> 405, (3072, 8192) 208.2 -> 207.9.
 //
 // Block order is XCD-aware: the row blocks that share a weight tile get block ids that are
 // equal modulo 8, so they run on one XCD and re-read the tile from its L2.
@@ -41,8 +41,96 @@ struct RopeOut {
   int S, Hq, Hk, L, HD;
 };
 
+// 128 x 128 with two stages, three workgroups per CU: their waves hide each other's loads and conversions,
+// where GemmTile reads ahead.  (Its products add k in another order: the other tiles agree bit for bit, with this one
+// in all but 0.1% of the values, and either is 2.07e-4 from float64.)  Wave w owns features 32 w .. + 31 of all 128 rows as 2 x 8 tiles of
+// v_mfma_f32_16x16x32_f16.  For launches of more than two workgroups per CU whose 256 x 128 tiles end in a half empty
+// round; us at 4096 rows, best of the other tiles -> this: (3072, 3072) 90.0 -> 79.7, (5120, 3072) 140 -> 132,
+// (3072, 8192) 218 -> 210.  (32x32x16 products in the same loop: 87.9, 145, 223.)
+template <bool RM>
+struct GemmTile3 : GemmTile<true, RM, 4, 1, 1, 4, 2> {
+  using G = GemmTile<true, RM, 4, 1, 1, 4, 2>;
+  static __device__ __forceinline__ void run(f16* lds, const f16* __restrict__ x, long ldx,
+                                             const int8_t* __restrict__ wp, const f16* __restrict__ sc, int M,
+                                             int N, int K, int n0, int m0) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nch = K >> 6, ntiles = (N + 15) >> 4;
+    const int t0 = min(n0 / 16, ntiles - 1);
+    const char* wb = (const char*)wp + (long)t0 * 16 * K;
+    const f16* xb = x;
+    uint32_t woff[2], xoff[4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int t = min(n0 / 16 + wv + 4 * j, ntiles - 1);
+      woff[j] = RM ? (uint32_t)((min(16 * t + (lane & 15), N - 1) - 16 * t0) * (long)K + 16 * (lane >> 4))
+                   : (uint32_t)((t - t0) * (16L * K)) + 16 * lane;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = 8 * (wv + 4 * j) + (lane >> 3);
+      xoff[j] = (uint32_t)(min(m0 + r, M - 1) * ldx * 2 + 16 * ((lane & 7) ^ (r & 7)));
+    }
+    const uint32_t lds0 = lds_addr(lds) + wv * 1024;
+    auto load = [&](int st) {
+      const uint32_t sa = lds0 + st * (G::STG * 2);
+      static_for<0, 2>([&](auto J) { lds_dma16_at<4096 * J.value>(wb, woff[J.value], sa); });
+      static_for<0, 4>([&](auto J) { lds_dma16_at<G::LW * 2 + 4096 * J.value>(xb, xoff[J.value], sa); });
+      wb += RM ? 64 : 1024;
+      xb += 64;
+    };
+    f16 scale[2];
+    f32x4 acc[2][8];
+#pragma unroll
+    for (int ft = 0; ft < 2; ++ft) {
+      scale[ft] = sc[min(n0 + 32 * wv + 16 * ft + (lane & 15), N - 1)];
+#pragma unroll
+      for (int rt = 0; rt < 8; ++rt) acc[ft][rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    load(0);
+    for (int c = 0; c < nch; ++c) {
+      wait_vm_lgkm0<0>();  // this wave's loads of chunk c, and its reads of chunk c - 1
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();  // chunk c complete; the stage of chunk c - 1 is free
+      asm volatile("" ::: "memory");
+      if (c + 1 < nch) load((c + 1) & 1);
+      const f16* st = lds + (c & 1) * G::STG;
+      f16x8 w[2][2];
+#pragma unroll
+      for (int ft = 0; ft < 2; ++ft) {
+        i8x16_to_f16(*(const u32x4*)(st + (2 * wv + ft) * 512 + 8 * lane), w[ft][0], w[ft][1]);
+        w[ft][0] = w[ft][0] * scale[ft];
+        w[ft][1] = w[ft][1] * scale[ft];
+      }
+#pragma unroll
+      for (int rt = 0; rt < 8; ++rt) {
+        const f16* xr = st + G::LW + (16 * rt + (lane & 15)) * 64;
+        f16x8 xv[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) xv[h] = *(const f16x8*)(xr + 8 * ((2 * (lane >> 4) + h) ^ (lane & 7)));
+#pragma unroll
+        for (int ft = 0; ft < 2; ++ft)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            acc[ft][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[ft][h], xv[h], acc[ft][rt], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ft = 0; ft < 2; ++ft)
+#pragma unroll
+      for (int rt = 0; rt < 8; ++rt) {
+        const int nl = 32 * wv + 16 * ft + 4 * (lane >> 4);
+        f16x4 yv;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) yv[j] = (f16)acc[ft][rt][j];
+        *(f16x4*)(lds + G::piece(16 * rt + (lane & 15), nl >> 3) + (nl & 4)) = yv;
+      }
+    __syncthreads();
+  }
+};
+
 template <int EPI, bool RM, int WN, int WM, int FT, int RT, int NS>
-__global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_kernel(
+__global__ __launch_bounds__(64 * WN * WM, NS == 2 ? 3 : 2) void gemm_i8p_kernel(
     const f16* __restrict__ x, long ldx, const int8_t* __restrict__ wp,
     const f16* __restrict__ s, const f16* __restrict__ res, long ldr, f16* __restrict__ y, long ldy,
     int M, int N, int K, int nfb, int nmb, RopeOut ro) {
@@ -52,7 +140,10 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_kernel(
   G::block(nfb, nmb, fb, mb);
   const int n0 = fb * G::BN, m0 = mb * G::BM;
   const RowMap rm = {0, 0, -1, 0, 0, 1, {0, 0, 0, 0, 0, 0, 0, 0}};  // plain rows
-  G::run(lds, x, ldx, wp, s, nullptr, M, N, K, n0, m0, rm);
+  if constexpr (NS == 2)
+    GemmTile3<RM>::run(lds, x, ldx, wp, s, M, N, K, n0, m0);
+  else
+    G::run(lds, x, ldx, wp, s, nullptr, M, N, K, n0, m0, rm);
   constexpr int U = G::U;
   const int p = threadIdx.x % G::PR, nb = n0 + 8 * p;
   if (nb >= N) return;
@@ -172,11 +263,25 @@ constexpr Tile TILES[4] = {
     {64, 64, 255, 280, 600},     // 4: 4 waves of 32 x 32, 12 stages
 };
 
-// The tile of the shortest estimate.  (Of 18 prompt shapes measured with every tile it is the fastest or
-// within 3% of it.)
+// 5: GemmTile3, from its third workgroup per CU up to three full rounds of 768; there only tile 1 is ever faster,
+// where its last round of 256 is nearly full (beyond, tile 1 always: (16384, 3072) at 3072 rows 296 us, at 4096 405,
+// tile 5 310 and 455).  A round of 768 takes 1550 ns a chunk, a last one of b workgroups 270 + 1260 b / 768; of tile 1
+// a round takes 980, a last one 520 + 460 b / 256.
+constexpr int THREE_PER_CU = 5;
+static bool three_per_cu(int M, int N, int nch) {
+  const long rows = (M + 127) / 128, b5 = (N + 127) / 128 * rows, b1 = (N + 255) / 256 * rows;
+  if (b5 <= 2 * 256 || b5 > 3 * 768 || !w_offsets_fit(128, nch)) return false;
+  const long last = b5 % 768;
+  const long e5 = b5 / 768 * (nch * 1550L + 2500) + (last ? nch * (270 + 1260 * last / 768) + 2500 : 0);
+  const long e1 = b1 / 256 * (nch * 980L + 2500) + (b1 % 256 ? nch * (520 + 460 * (b1 % 256) / 256) + 2500 : 0);
+  return e5 < e1;
+}
+
+// The tile of the shortest estimate.  (Of 18 prompt shapes of few rows measured with every tile it is the fastest or
+// within 3% of it, of 137 shapes of 300 to 4096 rows within 2%.)
 static int default_tile(int M, int N, int K) {
   long est = 0;
-  return 1 + best_tile(TILES, 4, M, N, K >> 6, 1, &est);
+  return three_per_cu(M, N, K >> 6) ? THREE_PER_CU : 1 + best_tile(TILES, 4, M, N, K >> 6, 1, &est);
 }
 
 // K split over gridDim.y: fp32 partial sums [gridDim.y][M, N]
@@ -207,15 +312,16 @@ static int launch_partial(const f16* x, long ldx, const int8_t* wp, const f16* s
 template <int EPI, bool RM = false>
 static int launch_gemm(const f16* x, long ldx, const int8_t* wp, const f16* s, const f16* res,
                        long ldr, f16* y, long ldy, int M, int N, int K, hipStream_t st,
-                       RopeOut ro = RopeOut{}) {
+                       RopeOut ro = RopeOut{}, int cfg = 0) {
 #define I8_CFG(I, ...)                                                                            \
   case I:                                                                                         \
     return launch_cfg<EPI, RM, __VA_ARGS__>(x, ldx, wp, s, res, ldr, y, ldy, M, N, K, st, ro)
-  switch (default_tile(M, N, K)) {
+  switch (cfg ? cfg : default_tile(M, N, K)) {
     I8_CFG(1, 8, 1, 1, 4, 3);
     I8_CFG(2, 4, 1, 1, 4, 3);
     I8_CFG(3, 2, 2, 1, 2, 7);
     I8_CFG(4, 2, 2, 1, 1, 12);
+    I8_CFG(5, 4, 1, 1, 4, 2);
     default: return ECD_EINVAL;
   }
 #undef I8_CFG
@@ -251,6 +357,24 @@ int ecd_gemm_i8p(const void* x, long ldx, const void* wp, const void* s, const v
   if (!x_offsets_fit(M, ldx)) return ECD_ENOTSUP;
   return launch_gemm<GEPI_STORE>((const f16*)x, ldx, (const int8_t*)wp, (const f16*)s,
                                  (const f16*)res, ldr, (f16*)y, ldy, M, N, K, (hipStream_t)stream);
+}
+
+int ecd_gemm_i8p_tile(int M, int N, int K) {
+  return M > 0 && N > 0 && K > 0 && K % 64 == 0 ? default_tile(M, N, K) : 0;
+}
+
+int ecd_gemm_i8p_tuned(const void* x, long ldx, const void* w, const void* s, const void* res, long ldr, void* y,
+                       long ldy, int M, int N, int K, int rowmajor, int cfg, void* stream) {
+  if (!x || !w || !s || !y || M <= 0 || N <= 0 || K <= 0 || (K % 64) || ldx < K || (ldx % 8) || !al16(x) ||
+      !al16(w) || ldy < N || (res && ldr < N) || cfg < 0 || cfg > 5)
+    return ECD_EINVAL;
+  if (!x_offsets_fit(M, ldx)) return ECD_ENOTSUP;
+  const f16 *xh = (const f16*)x, *sh = (const f16*)s, *rh = (const f16*)res;
+  const int8_t* wh = (const int8_t*)w;
+  const hipStream_t st = (hipStream_t)stream;
+  if (rowmajor)
+    return launch_gemm<GEPI_STORE, true>(xh, ldx, wh, sh, rh, ldr, (f16*)y, ldy, M, N, K, st, RopeOut{}, cfg);
+  return launch_gemm<GEPI_STORE>(xh, ldx, wh, sh, rh, ldr, (f16*)y, ldy, M, N, K, st, RopeOut{}, cfg);
 }
 
 int ecd_gemm_i8p_rope(const void* x, long ldx, const void* wp, const void* s, const float* rope,

@@ -383,6 +383,14 @@ int ecd_layer_stack(const void* plan, int nl, const void* o, const void* xin, co
 int ecd_gemm_i8p(const void* x, long ldx, const void* wp, const void* s, const void* res,
                  long ldr, void* y, long ldy, int M, int N, int K, void* stream);
 
+/* ecd_gemm_i8p (rowmajor 0: w = ecd_pack_i8(w)) or the dense int8_mm product (rowmajor 1: w [N, K] int8) with an
+ * explicit block tile (cfg 1..5: 256x128, 128x128, 64x128, 64x64 features x rows, then 128x128 with three workgroups
+ * per CU; 0 = the library's choice, which ecd_gemm_i8p_tile tells).  Replaces nothing in the reference: for sweeps
+ * and for the tests of every tile. */
+int ecd_gemm_i8p_tile(int M, int N, int K);
+int ecd_gemm_i8p_tuned(const void* x, long ldx, const void* w, const void* s, const void* res, long ldr, void* y,
+                       long ldy, int M, int N, int K, int rowmajor, int cfg, void* stream);
+
 /* The same GEMM on row-interleaved w1|w3 (ecd_pack_i8 with interleave) with the SiLU * mul
  * epilogue: mm[m, j] = fp16(fp16(silu(a_j)) * b_j), a/b the GEMM outputs of rows 2j / 2j + 1
  * (app/engine.py:152-153, app/kernels.py:171-180).  mm [M, F] (row stride ldm). */
