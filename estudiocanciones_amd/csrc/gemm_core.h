@@ -145,12 +145,13 @@ inline long tile_estimate(const Tile& t, int M, int N, int nch, int ks) {
 }
 
 // The loads' weight offsets are 32-bit from a workgroup's first feature: its bn features of K 16-bit values
-// (int8 weights: half of that) must stay below 4 GiB.
+// (int8 weights: half of that) must stay below 4 GiB.  A K for which even 64 features do not fit runs on 64 x 64 tiles
+// with a base of its own for every load (GemmTile::run's BIG).
 inline bool w_offsets_fit(int bn, int nch) { return (long)bn * nch * 128 <= 0xFFFFFFFFL; }
 
 // The tile of the shortest estimate (0-based) among those whose weight offsets fit, and that estimate.
 inline int best_tile(const Tile* t, int n, int M, int N, int nch, int ks, long* est) {
-  int best = n - 1;  // the narrowest: the launch refuses it if even that does not fit
+  int best = n - 1;
   *est = 0x7FFFFFFFFFFFFFFFL;
   for (int i = 0; i < n; ++i) {
     const long e = tile_estimate(t[i], M, N, nch, ks);
@@ -245,7 +246,8 @@ struct GemmTile {
   // [N, K] int8 matrix instead of packed tiles.  Ends with a barrier.
   // PART: only K chunks c0 .. c0 + cn - 1 (plain rows), whose fp32 sums go to part [M, N] (N % 4 == 0)
   // instead, straight from the registers.
-  template <bool PART = false>
+  // BIG: weights whose offsets from the first feature pass 32 bits; each DMA instruction keeps its own base.
+  template <bool PART = false, bool BIG = false>
   static __device__ __forceinline__ void run(f16* lds, const f16* __restrict__ x, long ldx,
                                              const void* __restrict__ wp, const f16* __restrict__ sc,
                                              const float* __restrict__ bias, int M, int N, int K,
@@ -266,11 +268,15 @@ struct GemmTile {
     const int t0 = min(n0 / 16, ntiles - 1);
     const char* wb = (const char*)wp + (long)t0 * tile_bytes;
     uint32_t woff[WI];
+    const char* wbig[BIG ? WI : 1];
 #pragma unroll
     for (int j = 0; j < WI; ++j) {
       const int i = wv + NW * j;
       const int t = min(n0 / 16 + (W8 ? i : i >> 1), ntiles - 1);
-      if constexpr (RM)  // the same lane order from rows of w: row lane & 15 (past N: the last), unit lane >> 4
+      if constexpr (BIG) {
+        wbig[j] = (const char*)wp + (long)t * tile_bytes + (W8 ? 0 : 1024 * (i & 1));
+        woff[j] = RM ? (uint32_t)((min(16 * t + (lane & 15), N - 1) - 16 * t) * (long)K + 16 * (lane >> 4)) : 16 * lane;
+      } else if constexpr (RM)  // the same lane order from rows of w: row lane & 15 (past N: the last), unit lane >> 4
         woff[j] = (uint32_t)((min(16 * t + (lane & 15), N - 1) - 16 * t0) * (long)K + 16 * (lane >> 4));
       else
         woff[j] = (uint32_t)((t - t0) * tile_bytes) + (W8 ? 0 : 1024 * (i & 1)) + 16 * lane;
@@ -313,6 +319,10 @@ struct GemmTile {
     auto next_chunk = [&]() {
       xb += 64;
       wb += RM ? 64 : 1024 * WPT;
+      if constexpr (BIG) {
+#pragma unroll
+        for (int j = 0; j < WI; ++j) wbig[j] += RM ? 64 : 1024 * WPT;
+      }
       if (rm.k && ++tc == rm.cpt) {
         tc = 0;
         ++tap;
@@ -324,7 +334,7 @@ struct GemmTile {
     auto dma = [&](auto J, uint32_t sa) {
       constexpr int j = decltype(J)::value;
       if constexpr (j < WI)
-        lds_dma16_at<NW * j * 1024>(wb, woff[j], sa);
+        lds_dma16_at<NW * j * 1024>(BIG ? wbig[BIG ? j : 0] : wb, woff[j], sa);
       else
         lds_dma16_at<LW * 2 + NW * (j - WI) * 1024>(xb, odd ? xoff1[j - WI] : xoff[j - WI], sa);
     };

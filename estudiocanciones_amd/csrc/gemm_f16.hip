@@ -33,7 +33,7 @@ struct RopeOut {
   int T, H, HD;
 };
 
-template <int EPI, int WN, int WM, int FT, int RT, int NS>
+template <int EPI, int WN, int WM, int FT, int RT, int NS, bool BIG>
 __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
     const f16* __restrict__ x, long ldx, const f16* __restrict__ wp,
     const float* __restrict__ bias, float alpha, const f16* res, long ldr,
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void gemm_f16w_kernel(
   int fb, mb;
   G::block(nfb, nmb, fb, mb);
   const int n0 = fb * G::BN, m0 = mb * G::BM;
-  G::run(lds, x, ldx, wp, nullptr, bias, M, N, K, n0, m0, rm);
+  G::template run<false, BIG>(lds, x, ldx, wp, nullptr, bias, M, N, K, n0, m0, rm);
   constexpr int U = G::U;
   const int p = threadIdx.x % G::PR, nb = n0 + 8 * p;
   if (nb >= N) return;
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void pack_f16_kernel(const f16* __restrict__ w
   *(u32x4*)(out + (tile * nch + c) * 1024 + 512 * h + 8 * l) = v;
 }
 
-template <int EPI, int WN, int WM, int FT, int RT, int NS>
+template <int EPI, int WN, int WM, int FT, int RT, int NS, bool BIG = false>
 static int launch_cfg(const f16* x, long ldx, const f16* wp, const float* bias, float alpha,
                       const f16* res, long ldr, f16* y, long ldy, int M, int N, int K,
                       const RowMap& rm, const RopeOut& ro, hipStream_t st) {
@@ -177,8 +177,11 @@ static int launch_cfg(const f16* x, long ldx, const f16* wp, const float* bias, 
   const int nfb = (N + BN - 1) / BN;
   const int nmb = (M + BM - 1) / BM;
   const long blocks = (long)nfb * nmb;
-  if (blocks > 0x7FFFFFFFL || !w_offsets_fit(32 * WN * FT, K >> 6)) return ECD_ENOTSUP;
-  hipLaunchKernelGGL((gemm_f16w_kernel<EPI, WN, WM, FT, RT, NS>), dim3((unsigned)blocks),
+  if (blocks > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  if constexpr (!BIG)
+    if (!w_offsets_fit(BN, K >> 6))
+      return launch_cfg<EPI, 2, 2, 1, 1, 8, true>(x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K, rm, ro, st);
+  hipLaunchKernelGGL((gemm_f16w_kernel<EPI, WN, WM, FT, RT, NS, BIG>), dim3((unsigned)blocks),
                      dim3(64 * WN * WM), 0, st, x, ldx, wp, bias, alpha, res, ldr, y, ldy, M, N, K,
                      nfb, nmb, rm, ro);
   return ecd_launch_status();
@@ -385,7 +388,7 @@ int ecd_gemm_f16p_prelu(const void* x, long ldx, const void* wp, const float* bi
 }
 
 int ecd_gemm_f16p_splits(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64)) return 1;
+  if (M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64) || !w_offsets_fit(TILES[6].bn, K >> 6)) return 1;
   return split_ways(TILES, 8, TILES + 6, 2, M, N, K >> 6);
 }
 

@@ -129,8 +129,8 @@ struct GemmTile3 : GemmTile<true, RM, 4, 1, 1, 4, 2> {
   }
 };
 
-template <int EPI, bool RM, int WN, int WM, int FT, int RT, int NS>
-__global__ __launch_bounds__(64 * WN * WM, NS == 2 ? 3 : 2) void gemm_i8p_kernel(
+template <int EPI, bool RM, int WN, int WM, int FT, int RT, int NS, bool BIG>
+__global__ __launch_bounds__(64 * WN * WM, 2) void gemm_i8p_kernel(
     const f16* __restrict__ x, long ldx, const int8_t* __restrict__ wp,
     const f16* __restrict__ s, const f16* __restrict__ res, long ldr, f16* __restrict__ y, long ldy,
     int M, int N, int K, int nfb, int nmb, RopeOut ro) {
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64 * WN * WM, NS == 2 ? 3 : 2) void gemm_i8p_kernel
   if constexpr (NS == 2)
     GemmTile3<RM>::run(lds, x, ldx, wp, s, M, N, K, n0, m0);
   else
-    G::run(lds, x, ldx, wp, s, nullptr, M, N, K, n0, m0, rm);
+    G::template run<false, BIG>(lds, x, ldx, wp, s, nullptr, M, N, K, n0, m0, rm);
   constexpr int U = G::U;
   const int p = threadIdx.x % G::PR, nb = n0 + 8 * p;
   if (nb >= N) return;
@@ -238,15 +238,18 @@ __global__ __launch_bounds__(64 * WN * WM, NS == 2 ? 3 : 2) void gemm_i8p_kernel
   }
 }
 
-template <int EPI, bool RM, int WN, int WM, int FT, int RT, int NS>
+template <int EPI, bool RM, int WN, int WM, int FT, int RT, int NS, bool BIG = false>
 static int launch_cfg(const f16* x, long ldx, const int8_t* wp, const f16* s, const f16* res,
                       long ldr, f16* y, long ldy, int M, int N, int K, hipStream_t st,
                       const RopeOut& ro) {
   constexpr int BN = 32 * WN * FT, BM = 32 * WM * RT;
   const int nfb = (N + BN - 1) / BN, nmb = (M + BM - 1) / BM;
   const long blocks = (long)nfb * nmb;
-  if (blocks > 0x7FFFFFFFL || !w_offsets_fit(32 * WN * FT, K >> 6)) return ECD_ENOTSUP;
-  hipLaunchKernelGGL((gemm_i8p_kernel<EPI, RM, WN, WM, FT, RT, NS>), dim3((unsigned)blocks),
+  if (blocks > 0x7FFFFFFFL) return ECD_ENOTSUP;
+  if constexpr (!BIG)
+    if (!w_offsets_fit(BN, K >> 6))
+      return launch_cfg<EPI, RM, 2, 2, 1, 1, 12, true>(x, ldx, wp, s, res, ldr, y, ldy, M, N, K, st, ro);
+  hipLaunchKernelGGL((gemm_i8p_kernel<EPI, RM, WN, WM, FT, RT, NS, BIG>), dim3((unsigned)blocks),
                      dim3(64 * WN * WM), 0, st, x, ldx, wp, s, res, ldr, y, ldy, M, N, K, nfb, nmb, ro);
   return ecd_launch_status();
 }
@@ -338,7 +341,7 @@ static bool x_offsets_fit(int M, long ldx) { return (long)M * ldx * 2 < 0x7FFFFF
 int gemm_i8_rowmajor(const f16* x, long ldx, const int8_t* w, const f16* s, const f16* res,
                      long ldr, f16* y, long ldy, int M, int N, int K, hipStream_t st) {
   if ((K % 64) || (ldx % 8) || !al16(x) || !al16(w) || !x_offsets_fit(M, ldx) ||
-      !w_offsets_fit(64, K >> 6))
+      16L * K >= 0x7FFFFFFFL)
     return 1;
   return launch_gemm<GEPI_STORE, true>(x, ldx, w, s, res, ldr, y, ldy, M, N, K, st);
 }
@@ -368,7 +371,7 @@ int ecd_gemm_i8p_tuned(const void* x, long ldx, const void* w, const void* s, co
   if (!x || !w || !s || !y || M <= 0 || N <= 0 || K <= 0 || (K % 64) || ldx < K || (ldx % 8) || !al16(x) ||
       !al16(w) || ldy < N || (res && ldr < N) || cfg < 0 || cfg > 5)
     return ECD_EINVAL;
-  if (!x_offsets_fit(M, ldx)) return ECD_ENOTSUP;
+  if (!x_offsets_fit(M, ldx) || (rowmajor && 16L * K >= 0x7FFFFFFFL)) return ECD_ENOTSUP;
   const f16 *xh = (const f16*)x, *sh = (const f16*)s, *rh = (const f16*)res;
   const int8_t* wh = (const int8_t*)w;
   const hipStream_t st = (hipStream_t)stream;
@@ -402,7 +405,7 @@ int ecd_gemm_i8p_silu(const void* x, long ldx, const void* wp, const void* s, vo
 }
 
 int ecd_gemm_i8p_splits(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64)) return 1;
+  if (M <= 0 || N <= 0 || K <= 0 || (K % 64) || (N % 64) || !w_offsets_fit(TILES[2].bn, K >> 6)) return 1;
   return split_ways(TILES, 4, TILES + 2, 2, M, N, K >> 6);
 }
 

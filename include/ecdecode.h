@@ -379,7 +379,7 @@ int ecd_layer_stack(const void* plan, int nl, const void* o, const void* xin, co
  * prompt pass (app/engine.py:123-153, 174-178).  MFMA-tiled, the tile by shape.
  *   x [M, K] fp16 (row stride ldx, 16-byte aligned, K % 64 == 0); wp = ecd_pack_i8(w);
  *   s [N] fp16; res [M, N] (row stride ldr) or NULL; y [M, N] (row stride ldy).
- *   ECD_ENOTSUP when M * ldx * 2 bytes reach 2 GiB or K exceeds 2^25 (32-bit per-lane load offsets). */
+ *   ECD_ENOTSUP when M * ldx * 2 bytes reach 2 GiB (32-bit per-lane load offsets). */
 int ecd_gemm_i8p(const void* x, long ldx, const void* wp, const void* s, const void* res,
                  long ldr, void* y, long ldy, int M, int N, int K, void* stream);
 
@@ -418,7 +418,7 @@ int ecd_gemm_i8p_rope(const void* x, long ldx, const void* wp, const void* s, co
  *   ecd_gemm_f16p_silu: w packed with interleave (gate | up), mm[m, j] =
  *                       fp16(fp16(silu(g)) * u) with g, u the fp16 GEMM outputs (LlamaMLP,
  *                       transformer.py:181-184).
- * x [M, K] fp16 (row stride ldx, 16-byte aligned, K % 64 == 0); ECD_ENOTSUP when K exceeds 2^25 or M * ldx * 2
+ * x [M, K] fp16 (row stride ldx, 16-byte aligned, K % 64 == 0); ECD_ENOTSUP when M * ldx * 2
  * bytes reach 2 GiB. */
 long ecd_packed_bytes_f16(int N, int K);
 int ecd_pack_f16(const void* w, int N, int K, int interleave, void* out, void* stream);
@@ -452,7 +452,7 @@ int ecd_gemm_f16p_conv(const void* x, long ldx, const void* wp, const float* bia
 
 /* A product of few rows split over K, for consumers that add the fp32 partial sums: ecd_gemm_*_splits gives
  * the number of ways (1: use the ordinary call), ecd_gemm_*_partial writes ws [ks][M, N] (N % 64 == 0,
- * ks <= 8, 16-byte aligned; no bias, scale or residual).  ecd_codec_norm_mod_sum is ecd_codec_norm_mod with
+ * ks <= 8, 16-byte aligned; no bias, scale or residual; ECD_ENOTSUP from K = 2^25, where the ways are 1).  ecd_codec_norm_mod_sum is ecd_codec_norm_mod with
  * h = fp16(sum of hp [ks][R, D] in order); ecd_rms_sum adds res, writes the sum to xo and its RMSNorm to y
  * (the reference's residual add and next norm, app/engine.py:141-153; D % 8 == 0, D <= 4096). */
 int ecd_gemm_f16p_splits(int M, int N, int K);
