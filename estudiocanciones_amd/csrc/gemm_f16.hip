@@ -207,11 +207,19 @@ constexpr Tile TILES[8] = {
 // tile 9 213 / 43, 5 228 / 62, 3 270 / 79; 1.4 M rows, 64 channels, K = 448 / 64: tile 10 274 / 69,
 // 9 295 / 91, 7 322 / 134).
 constexpr int MANY_ROWS = 16384;
+// Tile 10 also for short K (at most 8 chunks), where the fill of a deep ring is most of the time: up to one round of it,
+// and up to two where the 128 x 128 tiles need a second as well.  us, best of the others -> tile 10 (before this main
+// loop): 8000 x 256 x 256 6.70 -> 5.33 (6.11), 4500 x 256 x 256 6.37 -> 4.98 (5.81), 16000 x 128 x 128 5.89 -> 4.82
+// (5.63), 2000 x 1024 x 512 7.81 -> 6.54 (7.45), 3000 x 512 x 512 7.58 -> 6.25 (7.23), 20000 x 192 x 256 11.9 -> 8.9
+// (12.1), 1 x 256 x 256 4.40 -> 4.25 (3.80); with K = 1024 2000 x 1024 11.8 -> 13.0.
+constexpr int SHORT_K = 512;
 
 // Library default per shape (N counts output features before the SiLU pairing): the tile of the
 // shortest estimate.  (Of 29 shapes measured with every tile it is the fastest or within 10% of it.)
 static int default_cfg(int M, int N, int K) {
   if (M >= MANY_ROWS && N <= 128) return N <= 64 ? 10 : 9;
+  const long b10 = (long)((N + 63) / 64) * ((M + 127) / 128);
+  if (K <= SHORT_K && (b10 <= 256 || (b10 <= 512 && (long)((N + 127) / 128) * ((M + 127) / 128) > 256))) return 10;
   long est = 0;
   return 1 + best_tile(TILES, 8, M, N, K >> 6, 1, &est);
 }

@@ -98,3 +98,31 @@ def test_silu_rows_of_any_alignment(kind, F):
         buf, y = rows(M, F, ldy, lead)
         run(y, ldy)
         assert torch.equal(y, want) and gaps_kept(buf, y, lead, ldy)
+
+
+# the rule for short K: up to and past one round of 64 x 128 tiles, its second round where 128 x 128 tiles need one too,
+# the last K it takes and the first it does not, ragged rows and features
+@pytest.mark.parametrize("M,N,K", [(16384, 64, 64), (16385, 40, 64), (8193, 128, 512), (8193, 128, 576), (16256, 127, 128),
+                                   (16383, 128, 128), (8065, 193, 256), (4033, 513, 192),
+                                   (16500, 191, 64), (1, 64, 64)])
+def test_short_k_choice_equals_every_tile(M, N, K):
+    st = stream_ptr(torch.device("cuda"))
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randn(M, K, generator=g).half().cuda()
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).half().cuda()
+    b = torch.randn(N, generator=g).cuda()
+    wp, res = pack_f16(w), torch.randn(M, N, generator=g).half().cuda()
+
+    def run(cfg):
+        y = torch.empty(M, N, device="cuda", dtype=torch.float16)
+        _ffi.call("ecd_gemm_f16p_tuned", x.data_ptr(), K, wp.data_ptr(), b.data_ptr(), 0.25, res.data_ptr(), N, y.data_ptr(),
+                  N, M, N, K, 2, cfg, st)
+        return y
+
+    y = run(0)
+    assert all(torch.equal(y, run(cfg)) for cfg in (1, 5, 8, 9, 10))
+    v = x.double() @ w.double().t() + b.double()
+    want = torch.where(v < 0, 0.25 * v, v) + res.double()
+    # three fp16 roundings of values no larger than |v| + |res|, and K fp32 additions
+    tol = 3 * 2.0 ** -11 * (v.abs() + res.double().abs()) + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-6
+    assert bool(((y.double() - want).abs() <= tol).all())
