@@ -114,7 +114,7 @@ __device__ __forceinline__ void wait_vm() {
 __device__ __forceinline__ void wait_vm0() { wait_vm<0>(); }
 
 // LDS DMA, one wave instruction: 16 bytes per lane from base + off (base wave-uniform, off a
-// per-lane byte offset below 2^31) into LDS at dst + 16 * lane (dst uniform).  Issued from
+// per-lane byte offset, unsigned 32-bit) into LDS at dst + 16 * lane (dst uniform).  Issued from
 // inline asm with M0 (the instruction's LDS base) saved and restored around it: with the
 // compiler's builtin every later LDS read would wait for all outstanding DMA (vmcnt 0).
 // A vector instruction that writes a scalar register (readfirstlane, or the reload of a spilled one) needs

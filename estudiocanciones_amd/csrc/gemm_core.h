@@ -116,8 +116,8 @@ __device__ __forceinline__ int x_swz(int r) { return (r >> 1) & 7; }
 
 
 // fp16(silu(a)) * b for 4 interleaved pairs (a, b).  The sigmoid by the exp2 and reciprocal instructions (1 ulp
-// of fp32 each, against the 2^-11 of the rounding): with expf and an IEEE division the SiLU epilogue of
-// a 256 x 128 tile took about 5 us.
+// of fp32 each): for every finite fp16 a the rounded result is the nearest fp16, which expf and an IEEE division miss
+// once (a = -2.7246); with those the SiLU epilogue of a 256 x 128 tile took about 5 us.
 __device__ __forceinline__ f16x4 silu_mul4(const f16x8& v) {
   f16x4 o;
 #pragma unroll
@@ -165,7 +165,8 @@ inline int best_tile(const Tile* t, int n, int M, int N, int nch, int ks, long* 
 
 // Ways to split K for a product of few rows whose consumer adds fp32 partial sums (1: do not).  A split
 // launch fills CUs that the tiles of one leave idle, at most one workgroup per CU; the ks M N floats that it
-// writes and the consumer reads are taken at 2 floats per ps, its larger edges at 0.5 us.  Product and
+// writes and the consumer reads are taken at 2 ps each, its larger edges at 0.5 us.  (Its sums group K by the ways, so above
+// 64 rows the bits of a row depend on how many rows the call has; the decode attention's split is by rows too.)  Product and
 // consuming norm, us, one way -> the rule's ways (best of 1..8):
 //   fp16 weights  187 x 1536 x 1536   11.4 -> 10.1 (2)  10.1 | 187 x 1536 x 4096   17.4 -> 12.3 (3)  12.3
 //                 187 x 3072 x 8192   40.9 -> 28.5 (2)  28.5 | 187 x 3072 x 3072   16.5 -> 16.5 (1)  15.4

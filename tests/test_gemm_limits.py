@@ -26,14 +26,15 @@ def test_split_products_refuse_before_any_launch(K):
 # rows 48 .. 63 of the weights lie past 4 GiB from the first (fp16 6.4 GB of weights in all, int8 6.4 GB).  x is zero
 # but for a few values at both ends of K, so the product is a few exact terms.
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind", ["f16", "f16_wide_tile", "i8", "i8_rowmajor"])
+@pytest.mark.parametrize("kind", ["f16", "f16_wide_tile", "f16_below", "i8", "i8_rowmajor"])
 def test_weights_past_4_gib(kind):
     import torch
     from estudiocanciones_amd.kernels import gemm_f16_packed, gemm_packed, pack_f16, pack_i8, stream_ptr
     dev = torch.device("cuda:0")
     f16 = kind.startswith("f16")
     # the row-major product reads 16 rows from one base below 2 GiB (beyond, its own path): 64 of them pass 4 GiB too
-    K = 3 * 2 ** 24 if f16 else 2 ** 27 - 64 if kind == "i8_rowmajor" else 3 * 2 ** 25
+    # f16_below: the largest offsets lie between 2 and 4 GiB, the ordinary 64-feature tiles
+    K = 29 * 2 ** 20 if kind == "f16_below" else 3 * 2 ** 24 if f16 else 2 ** 27 - 64 if kind == "i8_rowmajor" else 3 * 2 ** 25
     M, N = (17 if kind == "i8_rowmajor" else 2), 66
     M = min(M, (2 ** 31 - 1) // (2 * K))
     at = [0, 5, 63, 64, K // 2, K - 65, K - 1]
@@ -48,7 +49,7 @@ def test_weights_past_4_gib(kind):
     if f16:
         wp = pack_f16(w)
         del w
-        if kind == "f16":
+        if kind != "f16_wide_tile":
             y = gemm_f16_packed(x, wp, N, K)
         else:
             y = torch.empty(M, N, device=dev, dtype=torch.float16)
