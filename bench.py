@@ -587,7 +587,7 @@ def main():
         prompt = {"prompt_tokens": P, "rows": B * P, "ms": round(p_ms, 3),
                   "gemm_flops": int(flops), "gemm_equivalent_TFLOPs": round(flops / p_ms / 1e9, 1),
                   "frac_of_mfma_f16_peak": round(flops / p_ms / 1e9 / 2500.0, 4),
-                  "path": ("MFMA GEMM (dense numerics, 2-stage LDS DMA) + MFMA causal flash "
+                  "path": ("MFMA GEMM (dense numerics, LDS DMA rings) + MFMA causal flash "
                           "attention, 28 layers")}
     codec = measure_codec(torch, dev, args.codec_steps, args.seed) if args.codec_steps > 0 else None
     traffic = None

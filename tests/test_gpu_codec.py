@@ -104,7 +104,7 @@ def test_gemm_f16_tile_configs_agree(dev, M, N, K, silu):
     xt, wp = D_(x, dev), pack_f16(D_(w, dev), interleave=bool(silu))
     No = N // 2 if silu else N
     outs = []
-    for cfg in range(0, 17):
+    for cfg in range(0, 17):  # ten tiles; the numbers 11 .. 16 are 1 .. 6 again, and stay accepted
         y = torch.empty(M, No, dtype=torch.float16, device=dev)
         _call("ecd_gemm_f16p_tuned", xt.data_ptr(), K, wp.data_ptr(),
               None if b is None else b.data_ptr(), 1.0 if silu else 0.75,
@@ -499,7 +499,7 @@ def test_gemm_f16_conv_implicit_taps(dev, offs, C, N, ypad, prelu, rep):
               y_imp.data_ptr(), N, y_imp.data_ptr(), N, B * T, N, K, T, P, ypad, off, k, rep, epi, st)
     _exact(N_(y_imp), N_(y_ref), f"implicit taps {offs} C={C} N={N} ypad={ypad} rep={rep}")
     # every block tile (sizes, LDS stages, pipelined or not) reads the implicit taps identically
-    for cfg in range(1, 17):
+    for cfg in range(1, 17):  # (11 .. 16: as 1 .. 6)
         y_cfg = D_(r, dev)
         _ffi.call("ecd_gemm_f16p_conv_tuned", xpt.data_ptr(), C, wp.data_ptr(), bt.data_ptr(), 0.25,
                   y_cfg.data_ptr(), N, y_cfg.data_ptr(), N, B * T, N, K, T, P, ypad, off, k, rep,
