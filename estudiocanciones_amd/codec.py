@@ -250,7 +250,8 @@ class LlamaTransformer:
 
     def _branch(self, lin, a, buf):
         """A residual branch's last linear layer (no bias) for the norm that adds it: fp16 rows, or with few
-        rows (fp32 partial sums, ways) of the product split over K."""
+        rows (fp32 partial sums, ways) of the product split over K.  The ways depend on the rows, so a short
+        window's low bits may differ alone and in a batch."""
         M, N = a.shape[0], lin.N
         ks = _ffi.lib().ecd_gemm_f16p_splits(M, N, lin.K)
         if ks == 1:

@@ -413,7 +413,8 @@ def gemm_packed(x, wp, s, N, K, res=None):
 def gemm_rms_packed(x, wp, s, N, K, res, nw, eps=1e-5):
     """(h, rms(h, nw)) with h = gemm_packed(x, wp, s, N, K, res): a residual branch and the next layer's
     norm.  With few rows the product is split over K and one kernel adds the fp32 partial sums and the
-    residual and forms the norm; the rounding points are the same."""
+    residual and forms the norm; the rounding points are the same.  The number of ways, and with it the
+    grouping of the fp32 sums, depends on M: a row's low bits may differ between calls of few and of many rows."""
     M = x.shape[0]
     ks = _ffi.lib().ecd_gemm_i8p_splits(M, N, K) if N <= 4096 and res.is_contiguous() and \
         res.data_ptr() % 16 == 0 and nw.data_ptr() % 16 == 0 else 1

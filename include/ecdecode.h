@@ -451,7 +451,7 @@ int ecd_gemm_f16p_conv(const void* x, long ldx, const void* wp, const float* bia
                        void* stream);
 
 /* A product of few rows split over K, for consumers that add the fp32 partial sums: ecd_gemm_*_splits gives
- * the number of ways (1: use the ordinary call), ecd_gemm_*_partial writes ws [ks][M, N] (N % 64 == 0,
+ * the number of ways for the shape (1: use the ordinary call), ecd_gemm_*_partial writes ws [ks][M, N] (N % 64 == 0,
  * ks <= 8, 16-byte aligned; no bias, scale or residual; ECD_ENOTSUP from K = 2^25, where the ways are 1).  ecd_codec_norm_mod_sum is ecd_codec_norm_mod with
  * h = fp16(sum of hp [ks][R, D] in order); ecd_rms_sum adds res, writes the sum to xo and its RMSNorm to y
  * (the reference's residual add and next norm, app/engine.py:141-153; D % 8 == 0, D <= 4096). */
