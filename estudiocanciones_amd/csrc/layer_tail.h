@@ -221,6 +221,11 @@ __device__ __forceinline__ void poll_pause(int it) {
 // is recognised from the go value the workgroup holds (all modulo 2^32; `per` divides 2^32).
 // Called by one lane after this workgroup's output stores have been acknowledged.
 constexpr int GATE_FLAGS = 1024;
+// The word a workgroup of group x takes its go value from at its start: its own group's flag.  All flags are equal
+// when a launch begins, but another group's may have moved on before a late workgroup (a cold first dispatch) looks: it
+// passes as soon as its 32 have arrived.  The own one waits for this workgroup.  The copy for group x + 1 is read, not one
+// in the lines that this group polls (the frame at KV 4096 1516 us either way before, 1520 with those).
+__device__ __forceinline__ constexpr int GATE_START(int x) { return GATE_FLAGS + 32 * (8 * ((x + 1) & 7) + x); }
 
 __device__ __forceinline__ void gate_arrive(uint32_t* sync, int grp, uint32_t per, uint32_t go) {
   if (add_agent(sync + 64 * (1 + grp)) == (go + 1u) * per - 1u) {
@@ -1720,7 +1725,7 @@ __global__ __launch_bounds__(NTHR) void layer_tail_kernel(const Args a) {
   }
   const bool ld0 = threadIdx.x == CW * 64;  // the loader's lane 0
   uint32_t go = 0, bad = 0;
-  if (ld0) go = ld_sc1(a.sync + GATE_FLAGS + 32 * 8 * (blockIdx.x & 7));  // (all flags equal here)
+  if (ld0) go = ld_sc1(a.sync + GATE_START(blockIdx.x & 7));
   tail_loader<CD, CF, NT13, KS2, AHD, AG, NTL, HEAD, R, VS, KNT, false>(a, smem, s_epoch, go, bad,
                                                                          false);
   if (ld0 && bad) flag_err(a.err, bad);
@@ -1782,7 +1787,7 @@ __global__ __launch_bounds__(NTHR) void layer_stack_kernel(const Args a0,
   }
   const bool ld0 = threadIdx.x == CW * 64;
   uint32_t go = 0, bad = 0;
-  if (ld0) go = ld_sc1(a0.sync + GATE_FLAGS + 32 * 8 * (blockIdx.x & 7));
+  if (ld0) go = ld_sc1(a0.sync + GATE_START(blockIdx.x & 7));
   auto layer = [&](int l) __attribute__((always_inline)) {
     tail_loader<CD, CF, NT13, KS2, AHD, AG, NTL, false, R, VS, KNT, true>(
         stack_args(plan, l), smem, s_epoch, go, bad, l > 0);
