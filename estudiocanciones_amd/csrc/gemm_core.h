@@ -136,7 +136,8 @@ struct Tile {
 };
 constexpr int LIGHT = 144;
 
-// Estimate of a launch over nch chunks, K split `ks` ways: rounds of 256 workgroups.
+// Estimate of a launch over nch chunks, K split `ks` ways: rounds of 256 workgroups (also for a tile of which two fit a
+// CU: their rounds run at the same time, each chunk twice as long).
 inline long tile_estimate(const Tile& t, int M, int N, int nch, int ks) {
   const long blocks = (long)((N + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm) * ks;
   const long load = blocks <= LIGHT ? 0 : (blocks >= 256 ? 256 - LIGHT : blocks - LIGHT);
